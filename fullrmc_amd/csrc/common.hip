@@ -1,6 +1,8 @@
 // common.hip -- error state, exact squared-norm thresholds, and the
 // boundary_conditions_collection entry points.
 #include <atomic>
+#include <mutex>
+#include <vector>
 #include <math.h>
 #include <stdarg.h>
 
@@ -63,6 +65,31 @@ hipError_t pool_malloc(void **p, size_t bytes, hipStream_t st) {
         retained.fetch_or(1ull << dev);
     }
     return hipMallocAsync(p, bytes, st);
+}
+
+static std::mutex g_words_mu;
+static std::vector<int64_t *> g_words_free;
+
+HostWords::HostWords(hipStream_t stream) : st(stream) {
+    {
+        std::lock_guard<std::mutex> lk(g_words_mu);
+        if (!g_words_free.empty()) {
+            p = g_words_free.back();
+            g_words_free.pop_back();
+            return;
+        }
+    }
+    if (hipHostMalloc((void **)&p, 16 * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+}
+
+HostWords::~HostWords() {
+    if (!p) return;
+    if (!waited) (void)hipStreamSynchronize(st);  // a kernel may still write them
+    std::lock_guard<std::mutex> lk(g_words_mu);
+    g_words_free.push_back(p);
 }
 
 int load_basis(const float *dbasis, Basis &B, bool &ortho, hipStream_t st) {

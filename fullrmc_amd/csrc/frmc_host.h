@@ -51,6 +51,24 @@ float sq_threshold(float t);
 // the driver at each synchronisation, so per-call scratch costs no mapping.
 hipError_t pool_malloc(void **p, size_t bytes, hipStream_t st);
 
+// Sixteen words of pinned host memory that a kernel of the call writes its
+// small results to: after the stream is waited for they can be read (a copy of
+// a few bytes to pageable memory instead costs 9 us more per call).  Taken from
+// a free list shared by all threads, returned at scope exit; the list is as
+// long as the most calls that ever ran at once.
+struct HostWords {
+    int64_t *p = nullptr;
+    hipStream_t st;
+    bool waited = false;
+    explicit HostWords(hipStream_t stream);
+    ~HostWords();
+    hipError_t wait() {
+        const hipError_t e = hipStreamSynchronize(st);
+        waited = e == hipSuccess;
+        return e;
+    }
+};
+
 // Basis / grid helpers (copy a device 3x3 to the host once per call).
 struct Basis;
 struct Grid;

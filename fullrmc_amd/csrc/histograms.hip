@@ -8,7 +8,8 @@
 //                  thread per (other atom), the list atoms uniform per block;
 //                  in-range pairs go straight to global int32 atomics (a
 //                  move touches O(g*N*fraction_in_range) bins).
-//  k_full_pairs    all unordered pairs i<j: triangular tile schedule, the
+//  k_full_pairs    all unordered pairs i<j, for the inputs and schedules that
+//                  the chunk pass (full_chunks.hip) does not take: triangular tile schedule, the
 //                  row atom in registers, the column tile staged in LDS
 //                  (float4 x,y,z,mol + elem), per-workgroup LDS-private bins
 //                  (2*nel^2*H int32) merged once into global counts.
@@ -21,13 +22,13 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <tuple>
 #include <vector>
 
-#include "frmc_device.h"
-#include "frmc_host.h"
+#include "full_hist.h"
 
 namespace frmc {
 
@@ -52,7 +53,8 @@ __global__ void k_fill_i32(int32_t *__restrict__ p, int64_t n, int32_t v) {
 
 // counts[0..size) -> hintra, counts[size..2size) -> hinter; add or overwrite
 __global__ void k_counts_to_float(const int32_t *__restrict__ counts, int64_t size, float *__restrict__ hintra,
-                                  float *__restrict__ hinter, int add) {
+                                  float *__restrict__ hinter, int add, int64_t *overflow) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *overflow = load_dev(counts + 2 * size);
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (; i < size; i += stride) {
@@ -82,23 +84,14 @@ __device__ __forceinline__ void count_pair(int32_t *__restrict__ counts, const H
 
 // ------------------------------------------------------------ multi coords
 
-// grid.x over other atoms i, grid.y over chunks of the index list.
+// One other atom i against the list's atoms c0..c1.
 template <bool PBC, bool ORTHO>
-__global__ void __launch_bounds__(256) k_multi_coords(const int32_t *__restrict__ indexes, int32_t nidx,
-                                                      int32_t per_block, const float *__restrict__ coords,
-                                                      int32_t n, const float *__restrict__ basis,
-                                                      const int32_t *__restrict__ mol,
-                                                      const int32_t *__restrict__ elem, HistArgs A, int allAtoms,
-                                                      int32_t *__restrict__ counts) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    Basis B;
-    bool ortho = false;
-    if (PBC) load_basis_dev(basis, B, ortho);
+__device__ __forceinline__ void multi_coords(const int32_t *__restrict__ indexes, int32_t c0, int32_t c1, int32_t i,
+                                             const float *__restrict__ coords, int32_t n, const Basis &B,
+                                             const int32_t *__restrict__ mol, const int32_t *__restrict__ elem,
+                                             const HistArgs &A, int allAtoms, int32_t *__restrict__ counts) {
     const float cx = coords[3 * (int64_t)i], cy = coords[3 * (int64_t)i + 1], cz = coords[3 * (int64_t)i + 2];
     int32_t mi = -1, ei = -1;
-    const int32_t c0 = blockIdx.y * per_block;
-    const int32_t c1 = min(nidx, c0 + per_block);
     for (int32_t c = c0; c < c1; c++) {
         const int32_t a = indexes[c];
         if (a < 0 || a >= n) continue;         // guarded; the host shim rejects such lists
@@ -113,6 +106,28 @@ __global__ void __launch_bounds__(256) k_multi_coords(const int32_t *__restrict_
         }
         count_pair(counts, A, s, elem[a], ei, mol[a] == mi);
     }
+}
+
+// grid.x over other atoms i, grid.y over chunks of the index list.  The cell's
+// kind is read here: reading the basis back first cost a synchronisation.
+template <bool PBC>
+__global__ void __launch_bounds__(256) k_multi_coords(const int32_t *__restrict__ indexes, int32_t nidx,
+                                                      int32_t per_block, const float *__restrict__ coords,
+                                                      int32_t n, const float *__restrict__ basis,
+                                                      const int32_t *__restrict__ mol,
+                                                      const int32_t *__restrict__ elem, HistArgs A, int allAtoms,
+                                                      int32_t *__restrict__ counts) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    Basis B;
+    bool ortho = false;
+    if (PBC) load_basis_dev(basis, B, ortho);
+    const int32_t c0 = blockIdx.y * per_block;
+    const int32_t c1 = min(nidx, c0 + per_block);
+    if (PBC && ortho)
+        multi_coords<PBC, true>(indexes, c0, c1, i, coords, n, B, mol, elem, A, allAtoms, counts);
+    else
+        multi_coords<PBC, false>(indexes, c0, c1, i, coords, n, B, mol, elem, A, allAtoms, counts);
 }
 
 // ------------------------------------------------------------- full pairs
@@ -133,68 +148,6 @@ struct FullSched {
 
 __host__ __device__ __forceinline__ int64_t row_block_start(int64_t bi, int64_t nct, int64_t R) {
     return bi * nct - R * bi * (bi - 1) / 2;
-}
-
-// Float64 edge re-check (EDGE mode): the histogram of the binary64 recompute
-// (every pair's distance evaluated in double from the float32 coordinates,
-// range and bin in double).  The float32 distance d32 of a pair is within
-// eps = 8u*(sum_m (|dx_m|+1)*rowsum_m + d32) of the double one (u = 2^-24;
-// error analysis of the float32 difference, the exact minimum-image
-// subtraction, the 3-term basis product, the squared norm and the rounded
-// sqrt, with a factor > 2 to spare); a pair whose d32 lies farther than eps
-// from every bin edge and range end, and whose fractional components are not
-// within a rounding tie of +-1/2, takes its bin from d32; every other pair is
-// recomputed in double.
-struct Edge64 {
-    double mn, mx, bn;      // the grid in double
-    float s_lo, s_hi;       // candidate window of float32 squared norms
-    float rowsum[3];        // sum_k |B[m][k]| per basis row (PBC), 1 otherwise
-};
-
-__device__ __forceinline__ double round64(double x) { return x > 0.0 ? floor(x + 0.5) : ceil(x - 0.5); }
-
-template <bool PBC>
-__device__ __forceinline__ double pair_d64(float ax, float ay, float az, float cx, float cy, float cz,
-                                           const Basis &B) {
-    const double dx = (double)ax - (double)cx, dy = (double)ay - (double)cy, dz = (double)az - (double)cz;
-    double rx = dx, ry = dy, rz = dz;
-    if (PBC) {
-        const double bx = dx - round64(dx), by = dy - round64(dy), bz = dz - round64(dz);
-        rx = (bx * (double)B.b[0] + by * (double)B.b[3]) + bz * (double)B.b[6];
-        ry = (bx * (double)B.b[1] + by * (double)B.b[4]) + bz * (double)B.b[7];
-        rz = (bx * (double)B.b[2] + by * (double)B.b[5]) + bz * (double)B.b[8];
-    }
-    return __builtin_sqrt((rx * rx + ry * ry) + rz * rz);
-}
-
-// Bin of a candidate pair in the binary64 recompute, or -1 out of range;
-// *rechecked is set when the pair needed the double evaluation.
-template <bool PBC>
-__device__ __forceinline__ int64_t edge_bin(float s, float ax, float ay, float az, float cx, float cy, float cz,
-                                            const Basis &B, const Edge64 &E, bool &rechecked) {
-    const float dx = ax - cx, dy = ay - cy, dz = az - cz;
-    const float d32 = cr_sqrt(s);
-    const float bound = (fabsf(dx) + 1.0f) * E.rowsum[0] + (fabsf(dy) + 1.0f) * E.rowsum[1] +
-                        (fabsf(dz) + 1.0f) * E.rowsum[2] + d32;
-    const double eps = 8.0 * 5.9604644775390625e-08 * 1.001 * (double)bound;
-    bool tie = false;
-    if (PBC) {
-        // fractional differences near +-1/2: float and double may pick different images
-        tie = fabsf(0.5f - fabsf(min_image(dx))) <= 4.8e-7f * (fabsf(dx) + 1.0f) ||
-              fabsf(0.5f - fabsf(min_image(dy))) <= 4.8e-7f * (fabsf(dy) + 1.0f) ||
-              fabsf(0.5f - fabsf(min_image(dz))) <= 4.8e-7f * (fabsf(dz) + 1.0f);
-    }
-    const double t = ((double)d32 - E.mn) / E.bn;
-    const double kf = floor(t);
-    const double margin = fmin(t - kf, kf + 1.0 - t) * E.bn;
-    rechecked = tie || margin <= eps || fabs((double)d32 - E.mn) <= eps || fabs((double)d32 - E.mx) <= eps;
-    if (rechecked) {
-        const double d = pair_d64<PBC>(ax, ay, az, cx, cy, cz, B);
-        if (d < E.mn || d >= E.mx) return -1;
-        return (int64_t)((d - E.mn) / E.bn);
-    }
-    if ((double)d32 < E.mn || (double)d32 >= E.mx) return -1;
-    return (int64_t)kf;
 }
 
 template <int NT, int R, bool PBC, bool ORTHO, bool LDS_HIST, bool EDGE>
@@ -284,7 +237,7 @@ __global__ void __launch_bounds__(NT) k_full_pairs(const float *__restrict__ coo
                     if (flat >= A.size) {
                         lost++;
                     } else if (LDS_HIST) {
-                        atomicAdd(&lds_hist[(intra ? 0 : size) + (int32_t)flat], 1);
+                        atomicAdd(&lds_hist[(intra ? size : 0) + (int32_t)flat], 1);
                     } else {
                         atomicAdd(&counts[(intra ? 0 : A.size) + flat], 1);
                     }
@@ -303,236 +256,6 @@ __global__ void __launch_bounds__(NT) k_full_pairs(const float *__restrict__ coo
     // EDGE: counts[2*size+1 .. +2] hold the number of double re-checks (64-bit, low word first)
     if (EDGE && tid == 0 && lds_rechecked)
         atomicAdd(reinterpret_cast<unsigned long long *>(&counts[2 * A.size + 2]), lds_rechecked);
-}
-
-// ------------------------------------------------ cell-list full histogram
-//
-// For periodic cells much larger than the histogram range, most pairs are
-// out of range.  The atoms are sorted into a grid of m0 x m1 x m2 fractional
-// cells, each at least the range (plus a margin) across: an atom's in-range
-// partners then lie in its own or the 26 neighbouring cells (the margin
-// covers the float32 rounding of the difference, image shift and norm).  A
-// work item is (cell c, one of 14 offsets: itself and 13 of the 26
-// neighbours, one of each opposite pair), so every unordered cell pair is
-// visited once; pairs whose cells are not neighbours are never evaluated and
-// count nowhere in either arithmetic.  Each pair keeps the reference's slot
-// [element(earlier index)][element(later index)] and intra/inter by molecule;
-// its distance is the same float32 (or binary64) value in either order.
-struct CellGrid {
-    int32_t m0, m1, m2;
-    int64_t ncell;
-    int64_t items;      // 14 per cell
-    int64_t per_block;  // items per workgroup
-};
-
-__device__ __forceinline__ int32_t cell_of(float x, int32_t m) {
-    const float f = x - floorf(x);  // exact: the fraction of a float
-    const int32_t c = (int32_t)(f * (float)m);
-    return c < 0 ? 0 : (c >= m ? m - 1 : c);
-}
-
-__global__ void __launch_bounds__(256) k_cell_count(const float *__restrict__ coords, int32_t n, CellGrid G,
-                                                    int32_t *__restrict__ cid, int32_t *__restrict__ cnt) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int32_t cx = cell_of(coords[3 * (int64_t)i], G.m0), cy = cell_of(coords[3 * (int64_t)i + 1], G.m1),
-                  cz = cell_of(coords[3 * (int64_t)i + 2], G.m2);
-    const int32_t c = (cx * G.m1 + cy) * G.m2 + cz;
-    cid[i] = c;
-    atomicAdd(&cnt[c], 1);
-}
-
-// exclusive scan of ncell counts into start[0..ncell] (one block); fill <- start
-__global__ void __launch_bounds__(1024) k_cell_scan(const int32_t *__restrict__ cnt, int64_t ncell,
-                                                    int32_t *__restrict__ start, int32_t *__restrict__ fill) {
-    __shared__ int32_t part[1024];
-    const int t = threadIdx.x;
-    const int64_t per = (ncell + 1023) / 1024;
-    const int64_t c0 = t * per, c1 = min(ncell, c0 + per);
-    int32_t sum = 0;
-    for (int64_t c = c0; c < c1; c++) sum += cnt[c];
-    part[t] = sum;
-    __syncthreads();
-    if (t == 0) {
-        int32_t acc = 0;
-        for (int q = 0; q < 1024; q++) {
-            const int32_t v = part[q];
-            part[q] = acc;
-            acc += v;
-        }
-        start[ncell] = acc;
-    }
-    __syncthreads();
-    int32_t acc = part[t];
-    for (int64_t c = c0; c < c1; c++) {
-        start[c] = acc;
-        fill[c] = acc;
-        acc += cnt[c];
-    }
-}
-
-// cell-sorted copies: (x, y, z, molecule bits), element, original index
-__global__ void __launch_bounds__(256) k_cell_scatter(const float *__restrict__ coords, int32_t n,
-                                                      const int32_t *__restrict__ mol,
-                                                      const int32_t *__restrict__ elem,
-                                                      const int32_t *__restrict__ cid, int32_t *__restrict__ fill,
-                                                      float4 *__restrict__ sx, int32_t *__restrict__ se,
-                                                      int32_t *__restrict__ sid) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int32_t pos = atomicAdd(&fill[cid[i]], 1);
-    sx[pos] = make_float4(coords[3 * (int64_t)i], coords[3 * (int64_t)i + 1], coords[3 * (int64_t)i + 2],
-                          __int_as_float(mol[i]));
-    se[pos] = elem[i];
-    sid[pos] = i;
-}
-
-// offset o of the 14 visited per cell: 0 the cell itself, 1..13 the
-// neighbours (dx, dy, dz) with dx > 0, or dx == 0 and dy > 0, or dx == dy == 0
-// and dz > 0
-__device__ __forceinline__ void cell_offset(int32_t o, int32_t &dx, int32_t &dy, int32_t &dz) {
-    if (o == 0) {
-        dx = dy = dz = 0;
-        return;
-    }
-    if (o <= 9) {  // dx = 1: the 9 (dy, dz)
-        dx = 1;
-        dy = (o - 1) / 3 - 1;
-        dz = (o - 1) % 3 - 1;
-    } else if (o <= 12) {  // dx = 0, dy = 1
-        dx = 0;
-        dy = 1;
-        dz = o - 11;
-    } else {  // dx = dy = 0, dz = 1
-        dx = 0;
-        dy = 0;
-        dz = 1;
-    }
-}
-
-// NT threads, up to R rows per thread per pass (a cell of more than R*NT
-// atoms takes several passes); LDS_HIST: workgroup-private bins as in
-// k_full_pairs, written to this workgroup's partial at the end.
-template <int NT, int R, bool ORTHO, bool LDS_HIST, bool EDGE>
-__global__ void __launch_bounds__(NT) k_full_cells(const float4 *__restrict__ sx, const int32_t *__restrict__ se,
-                                                    const int32_t *__restrict__ sid,
-                                                    const int32_t *__restrict__ cstart, CellGrid G, Basis B,
-                                                    HistArgs A, Edge64 E, int32_t *__restrict__ partial,
-                                                    int32_t *__restrict__ counts) {
-    extern __shared__ int32_t lds_hist[];
-    __shared__ float4 tile_x[NT];
-    __shared__ int32_t tile_e[NT], tile_id[NT];
-    __shared__ int32_t lds_overflow;
-    __shared__ unsigned long long lds_rechecked;
-    const int tid = threadIdx.x;
-    const int32_t size = (int32_t)A.size;
-    if (LDS_HIST)
-        for (int32_t s = tid; s < 2 * size; s += NT) lds_hist[s] = 0;
-    if (tid == 0) {
-        lds_overflow = 0;
-        lds_rechecked = 0;
-    }
-    const int64_t it0 = (int64_t)blockIdx.x * G.per_block;
-    const int64_t it1 = min(G.items, it0 + G.per_block);
-    int32_t lost = 0;
-    uint32_t nre = 0;
-    for (int64_t item = it0; item < it1; item++) {
-        const int64_t c = item / 14;
-        const int32_t o = (int32_t)(item % 14);
-        const int32_t cx = (int32_t)(c / ((int64_t)G.m1 * G.m2)), cy = (int32_t)((c / G.m2) % G.m1),
-                      cz = (int32_t)(c % G.m2);
-        int32_t dx, dy, dz;
-        cell_offset(o, dx, dy, dz);
-        const int64_t c2 = ((int64_t)((cx + dx + G.m0) % G.m0) * G.m1 + (cy + dy + G.m1) % G.m1) * G.m2 +
-                           (cz + dz + G.m2) % G.m2;
-        const bool self = o == 0;
-        const int32_t r0 = cstart[c], r1 = cstart[c + 1], q0 = cstart[c2], q1 = cstart[c2 + 1];
-        for (int32_t rp = r0; rp < r1; rp += NT * R) {
-            float rx[R], ry[R], rz[R];
-            int32_t rm[R], re[R], ri[R], rpos[R];
-#pragma unroll
-            for (int k = 0; k < R; k++) {
-                rpos[k] = rp + tid + NT * k;
-                const int32_t pr = min(rpos[k], r1 - 1);  // clamped; rows past the cell never count
-                const float4 v = sx[pr];
-                rx[k] = v.x;
-                ry[k] = v.y;
-                rz[k] = v.z;
-                rm[k] = __float_as_int(v.w);
-                re[k] = se[pr];
-                ri[k] = sid[pr];
-            }
-            for (int32_t tq = q0; tq < q1; tq += NT) {
-                __syncthreads();  // previous tile consumed
-                {
-                    const int32_t j = min(tq + tid, q1 - 1);
-                    tile_x[tid] = sx[j];
-                    tile_e[tid] = se[j];
-                    tile_id[tid] = sid[j];
-                }
-                __syncthreads();
-                const int32_t jn = min(NT, q1 - tq);
-#pragma unroll 2
-                for (int32_t t = 0; t < jn; t++) {
-                    const float4 q = tile_x[t];
-                    const int32_t ej = tile_e[t], idj = tile_id[t];
-#pragma unroll
-                    for (int k = 0; k < R; k++) {
-                        const float s = pair_s<true, ORTHO>(rx[k], ry[k], rz[k], q.x, q.y, q.z, B);
-                        const bool cand = EDGE ? (s >= E.s_lo && s < E.s_hi) : in_range(s, A.g);
-                        const bool ok = cand && rpos[k] < r1 && (!self || tq + t > rpos[k]);
-                        if (ok) {
-                            // the earlier atom is the reference's atomIndex: its element first
-                            const bool rfirst = ri[k] < idj;
-                            int64_t b;
-                            if (EDGE) {
-                                bool re64 = false;
-                                b = rfirst ? edge_bin<true>(s, rx[k], ry[k], rz[k], q.x, q.y, q.z, B, E, re64)
-                                           : edge_bin<true>(s, q.x, q.y, q.z, rx[k], ry[k], rz[k], B, E, re64);
-                                nre += re64;
-                                if (b < 0) continue;
-                            } else {
-                                b = bin_of(s, A.g);
-                            }
-                            const int32_t ea = rfirst ? re[k] : ej, eb = rfirst ? ej : re[k];
-                            const int64_t flat = ((int64_t)ea * A.nel + eb) * A.g.H + b;
-                            const bool intra = __float_as_int(q.w) == rm[k];
-                            if (flat >= A.size) {
-                                lost++;
-                            } else if (LDS_HIST) {
-                                atomicAdd(&lds_hist[(intra ? 0 : size) + (int32_t)flat], 1);
-                            } else {
-                                atomicAdd(&counts[(intra ? 0 : A.size) + flat], 1);
-                            }
-                        }
-                    }
-                }
-            }
-        }
-    }
-    if (lost) atomicAdd(&lds_overflow, lost);
-    if (EDGE && nre) atomicAdd(&lds_rechecked, (unsigned long long)nre);
-    __syncthreads();
-    if (LDS_HIST) {
-        int32_t *dst = partial + (int64_t)blockIdx.x * 2 * size;
-        for (int32_t s = tid; s < 2 * size; s += NT) dst[s] = lds_hist[s];
-    }
-    if (tid == 0 && lds_overflow) atomicAdd(&counts[2 * A.size], lds_overflow);
-    if (EDGE && tid == 0 && lds_rechecked)
-        atomicAdd(reinterpret_cast<unsigned long long *>(&counts[2 * A.size + 2]), lds_rechecked);
-}
-
-// counts[s] += sum over the workgroup partials p in this split of partial[p][s]
-__global__ void __launch_bounds__(256) k_sum_partials(const int32_t *__restrict__ partial, int32_t nparts,
-                                                      int64_t len, int32_t per_split,
-                                                      int32_t *__restrict__ counts) {
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= len) return;
-    const int32_t p0 = blockIdx.y * per_split;
-    const int32_t p1 = min(nparts, p0 + per_split);
-    int32_t acc = 0;
-    for (int32_t p = p0; p < p1; p++) acc += partial[(int64_t)p * len + s];
-    if (acc) atomicAdd(&counts[s], acc);
 }
 
 // --------------------------------------------------------------- from dists
@@ -596,35 +319,33 @@ static int alloc_counts(Scratch &sc, int64_t size, hipStream_t st) {
 }
 
 static int finish_counts(Scratch &sc, int64_t size, float *hintra, float *hinter, int add, hipStream_t st) {
+    HostWords ov(st);
+    if (!ov.p) {
+        set_error("allocation of pinned host words failed");
+        return FRMC_ENOMEM;
+    }
     unsigned g = blocks_for(size, 256);
     if (g > 2048) g = 2048;
-    k_counts_to_float<<<g, 256, 0, st>>>(sc.p, size, hintra, hinter, add);
+    k_counts_to_float<<<g, 256, 0, st>>>(sc.p, size, hintra, hinter, add, ov.p);
     FRMC_CHECK_LAUNCH();
-    int32_t ov = 0;
-    FRMC_CHECK_HIP(hipMemcpyAsync(&ov, sc.p + 2 * size, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    FRMC_CHECK_HIP(hipStreamSynchronize(st));
-    set_overflow(ov);
+    FRMC_CHECK_HIP(ov.wait());
+    set_overflow(ov.p[0]);
     return FRMC_OK;
 }
 
 static int launch_multi(const int32_t *indexes, int32_t nidx, const float *coords, int32_t n, const float *basis,
                         int isPBC, const int32_t *mol, const int32_t *elem, const HistArgs &A, int allAtoms,
-                        int32_t *counts, hipStream_t st, bool ortho_hint) {
+                        int32_t *counts, hipStream_t st) {
     if (nidx == 0 || n == 0) return FRMC_OK;
     const int32_t per_block = 16;
     dim3 grid(blocks_for(n, 256), (unsigned)((nidx + per_block - 1) / per_block));
     FRMC_REQUIRE(grid.y <= 65535, "index list too long (%d)", nidx);
-    if (isPBC) {
-        if (ortho_hint)
-            k_multi_coords<true, true><<<grid, 256, 0, st>>>(indexes, nidx, per_block, coords, n, basis, mol, elem,
-                                                             A, allAtoms, counts);
-        else
-            k_multi_coords<true, false><<<grid, 256, 0, st>>>(indexes, nidx, per_block, coords, n, basis, mol,
-                                                              elem, A, allAtoms, counts);
-    } else {
-        k_multi_coords<false, false><<<grid, 256, 0, st>>>(indexes, nidx, per_block, coords, n, basis, mol, elem, A,
-                                                           allAtoms, counts);
-    }
+    if (isPBC)
+        k_multi_coords<true><<<grid, 256, 0, st>>>(indexes, nidx, per_block, coords, n, basis, mol, elem, A, allAtoms,
+                                                   counts);
+    else
+        k_multi_coords<false><<<grid, 256, 0, st>>>(indexes, nidx, per_block, coords, n, basis, mol, elem, A, allAtoms,
+                                                    counts);
     FRMC_CHECK_LAUNCH();
     return FRMC_OK;
 }
@@ -684,10 +405,10 @@ static FullSched full_sched(int32_t n, int32_t nt, int32_t R, int64_t blocks) {
 // counts (integer atomics), so the choice only changes the time.
 struct FullChoice {
     int32_t nt = 256, R = 2, per_cu = 2;
-    bool cells = false;  // the cell-list kernel (R = 1024 / nt rows per thread per pass)
+    bool cells = false;  // asked for as the cell list: the chunk pass, on cells of three ranges and more
 };
 
-// Cells per axis for pairs up to maxR apart in the periodic cell B: each
+// The condition of a forced cell-list schedule.  Cells per axis for pairs up to maxR apart in the periodic cell B: each
 // axis gets floor(h / w) cells, h the spacing of the cell's lattice planes
 // across it and w = maxR (1 + 1e-5) + 0.01 A (the margin covers the float32
 // rounding of a pair's difference, image shift and norm).  False when an
@@ -737,17 +458,13 @@ static thread_local FullChoice g_last;     // frmc_last_full_schedule (per threa
 static thread_local int64_t g_last_blocks = 0;
 static thread_local int g_last_tuned = 0;
 static thread_local int64_t g_last_evaluated = -1;  // pairs evaluated by the last call (-1: not measured)
-static thread_local int64_t g_cells_evaluated = -1;  // set by run_cells when timing is on
+static thread_local int64_t g_chunks_evaluated = -1;  // set by run_chunks when timing is on
 static std::mutex g_tune_mu;
 // shape class -> tuned schedule.  Class: device, floor(log2 n), bins
 // (2*nel*nel*H), boundary kind (0 none, 1 triclinic, 2 orthorhombic), EDGE.
 static std::map<std::tuple<int, int, int64_t, int, int>, FullChoice> g_tuned;
 
 // One full-histogram pass with schedule C: counts += all pairs' bins.
-static int run_cells(const FullChoice &C, const float *coords, int32_t n, const Basis &B, bool ortho,
-                     const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E, int ncu,
-                     int32_t *counts, hipStream_t st, int64_t *nblocks);
-
 static double range_of(const HistArgs &A, const Edge64 *E) {
     return E ? sqrt((double)E->s_hi) : (double)A.g.maxD;
 }
@@ -755,7 +472,23 @@ static double range_of(const HistArgs &A, const Edge64 *E) {
 static int run_full(const FullChoice &C, const float *coords, int32_t n, const Basis &B, int isPBC, bool ortho,
                     const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E, int ncu,
                     int32_t *counts, hipStream_t st, int64_t *nblocks) {
-    if (C.cells) return run_cells(C, coords, n, B, ortho, mol, elem, A, E, ncu, counts, st, nblocks);
+    if (C.cells) {
+        int32_t m[3];
+        if (!isPBC || !cell_grid(B, range_of(A, E), m)) {
+            set_error("cell-list schedule on a cell too small for three cells per axis");
+            return FRMC_EINVAL;
+        }
+    }
+    if (C.cells && chunks_take(n, A)) {
+        ChunkRun R;
+        R.nt = C.nt;
+        R.per_cu = C.per_cu;
+        R.blocks = nblocks;
+        R.pairs = &g_chunks_evaluated;
+        R.counts = counts;
+        g_chunks_evaluated = -1;
+        return run_chunks(R, coords, n, nullptr, B, isPBC, mol, elem, A, E, ncu, st);
+    }
     const size_t lds_bytes = sizeof(int32_t) * 2 * A.size;
     const bool lds = lds_bytes <= kMaxLdsHistBytes;
     const FullSched S = full_sched(n, C.nt, C.R, (int64_t)ncu * C.per_cu);
@@ -791,136 +524,8 @@ static int run_full(const FullChoice &C, const float *coords, int32_t n, const B
     FRMC_FULL_CASE(1024, 4)
 #undef FRMC_FULL_CASE
     if (rc == FRMC_EINVAL) set_error("no full-histogram kernel for %d threads and %d row atoms", C.nt, C.R);
-    if (rc == FRMC_OK && lds) {
-        const int32_t per_split = 16;
-        const int64_t len = 2 * A.size;
-        dim3 grid(blocks_for(len, 256), (unsigned)((blocks + per_split - 1) / per_split));
-        k_sum_partials<<<grid, 256, 0, st>>>(partial, (int32_t)blocks, len, per_split, counts);
-        hipError_t le = hipGetLastError();
-        if (le != hipSuccess) {
-            set_error("k_sum_partials launch failed: %s", hipGetErrorString(le));
-            rc = FRMC_EHIP;
-        }
-    }
+    if (rc == FRMC_OK && lds) rc = add_partials(partial, blocks, A.size, counts, st);
     if (partial) (void)hipFreeAsync(partial, st);
-    return rc;
-}
-
-// The cell-list pass: sort the atoms into the cell grid (count, scan,
-// scatter), then k_full_cells over (cell, offset) items and the partials'
-// sum.  The caller checked cell_grid().
-static int run_cells(const FullChoice &C, const float *coords, int32_t n, const Basis &B, bool ortho,
-                     const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E, int ncu,
-                     int32_t *counts, hipStream_t st, int64_t *nblocks) {
-    int32_t m[3];
-    if (!cell_grid(B, range_of(A, E), m)) {
-        set_error("cell-list schedule on a cell too small for three cells per axis");
-        return FRMC_EINVAL;
-    }
-    CellGrid G;
-    G.m0 = m[0];
-    G.m1 = m[1];
-    G.m2 = m[2];
-    G.ncell = (int64_t)m[0] * m[1] * m[2];
-    G.items = 14 * G.ncell;
-    int64_t blocks = std::min<int64_t>(G.items, (int64_t)ncu * C.per_cu);
-    G.per_block = (G.items + blocks - 1) / blocks;
-    blocks = (G.items + G.per_block - 1) / G.per_block;
-    if (nblocks) *nblocks = blocks;
-    const size_t lds_bytes = sizeof(int32_t) * 2 * A.size;
-    const bool lds = lds_bytes <= kMaxLdsHistBytes;
-    // scratch: cell of each atom, cell counts / fill cursors / starts, the
-    // sorted atoms, then the workgroup partials
-    const size_t nn = (size_t)(n > 0 ? n : 1), nc = (size_t)G.ncell;
-    const size_t off_cnt = 16 * nn, off_fill = off_cnt + 4 * nc, off_start = off_fill + 4 * nc,
-                 off_se = (off_start + 4 * (nc + 1) + 15) & ~(size_t)15, off_sid = off_se + 4 * nn,
-                 off_cid = off_sid + 4 * nn, off_part = (off_cid + 4 * nn + 255) & ~(size_t)255;
-    const size_t bytes = off_part + (lds ? lds_bytes * (size_t)blocks : 0);
-    char *scr = nullptr;
-    hipError_t e = pool_malloc((void **)&scr, bytes, st);
-    if (e != hipSuccess) {
-        set_error("hipMallocAsync of %zu bytes for the cell-list histogram failed: %s", bytes, hipGetErrorString(e));
-        return FRMC_ENOMEM;
-    }
-    float4 *sx = (float4 *)scr;
-    int32_t *cnt = (int32_t *)(scr + off_cnt), *fill = (int32_t *)(scr + off_fill),
-            *cstart = (int32_t *)(scr + off_start), *se = (int32_t *)(scr + off_se), *sid = (int32_t *)(scr + off_sid),
-            *cid = (int32_t *)(scr + off_cid), *partial = lds ? (int32_t *)(scr + off_part) : nullptr;
-    k_fill_i32<<<blocks_for((int64_t)nc, 256), 256, 0, st>>>(cnt, (int64_t)nc, 0);
-    k_cell_count<<<blocks_for(n, 256), 256, 0, st>>>(coords, n, G, cid, cnt);
-    k_cell_scan<<<1, 1024, 0, st>>>(cnt, G.ncell, cstart, fill);
-    k_cell_scatter<<<blocks_for(n, 256), 256, 0, st>>>(coords, n, mol, elem, cid, fill, sx, se, sid);
-    hipError_t le = hipGetLastError();
-    g_cells_evaluated = -1;
-    if (le == hipSuccess && timing_enabled()) {
-        // pairs the items visit: n_c (n_c - 1) / 2 within a cell, n_c n_c' for
-        // each of its 13 visited neighbours (measurement only: synchronises)
-        std::vector<int32_t> hs(nc + 1);
-        le = hipMemcpyAsync(hs.data(), cstart, sizeof(int32_t) * (nc + 1), hipMemcpyDeviceToHost, st);
-        if (le == hipSuccess) le = hipStreamSynchronize(st);
-        if (le == hipSuccess) {
-            int64_t ev = 0;
-            for (int32_t x = 0; x < m[0]; x++)
-                for (int32_t y = 0; y < m[1]; y++)
-                    for (int32_t z = 0; z < m[2]; z++) {
-                        const int64_t c = ((int64_t)x * m[1] + y) * m[2] + z;
-                        const int64_t nc0 = hs[c + 1] - hs[c];
-                        ev += nc0 * (nc0 - 1) / 2;
-                        for (int32_t o = 1; o < 14; o++) {
-                            const int32_t dx = o <= 9 ? 1 : 0, dy = o <= 9 ? (o - 1) / 3 - 1 : (o <= 12 ? 1 : 0),
-                                          dz = o <= 9 ? (o - 1) % 3 - 1 : (o <= 12 ? o - 11 : 1);
-                            const int64_t c2 = ((int64_t)((x + dx + m[0]) % m[0]) * m[1] + (y + dy + m[1]) % m[1]) *
-                                                   m[2] + (z + dz + m[2]) % m[2];
-                            ev += nc0 * (hs[c2 + 1] - hs[c2]);
-                        }
-                    }
-            g_cells_evaluated = ev;
-        }
-    }
-    Edge64 none;
-    memset(&none, 0, sizeof(none));
-    const Edge64 &EE = E ? *E : none;
-    const size_t shm = lds ? lds_bytes : 0;
-#define FRMC_CELLS_LAUNCH(NT_, O, L, ED)                                                                        \
-    do {                                                                                                        \
-        if (shm > 48 * 1024)                                                                                    \
-            (void)hipFuncSetAttribute((const void *)k_full_cells<NT_, 1024 / NT_, O, L, ED>,                    \
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);                    \
-        k_full_cells<NT_, 1024 / NT_, O, L, ED><<<(unsigned)blocks, NT_, shm, st>>>(sx, se, sid, cstart, G, B, \
-                                                                                    A, EE, partial, counts);    \
-    } while (0)
-#define FRMC_CELLS_NT(NT_)                                                                                      \
-    do {                                                                                                        \
-        if (ortho) {                                                                                            \
-            if (lds) { if (E) FRMC_CELLS_LAUNCH(NT_, true, true, true); else FRMC_CELLS_LAUNCH(NT_, true, true, false); } \
-            else     { if (E) FRMC_CELLS_LAUNCH(NT_, true, false, true); else FRMC_CELLS_LAUNCH(NT_, true, false, false); } \
-        } else {                                                                                                \
-            if (lds) { if (E) FRMC_CELLS_LAUNCH(NT_, false, true, true); else FRMC_CELLS_LAUNCH(NT_, false, true, false); } \
-            else     { if (E) FRMC_CELLS_LAUNCH(NT_, false, false, true); else FRMC_CELLS_LAUNCH(NT_, false, false, false); } \
-        }                                                                                                       \
-    } while (0)
-    int rc = FRMC_OK;
-    if (le == hipSuccess) {
-        if (C.nt == 256) FRMC_CELLS_NT(256);
-        else if (C.nt == 512) FRMC_CELLS_NT(512);
-        else rc = FRMC_EINVAL;
-        le = hipGetLastError();
-    }
-#undef FRMC_CELLS_NT
-#undef FRMC_CELLS_LAUNCH
-    if (rc == FRMC_EINVAL) set_error("no cell-list kernel for %d threads", C.nt);
-    if (rc == FRMC_OK && le == hipSuccess && lds) {
-        const int32_t per_split = 16;
-        const int64_t len = 2 * A.size;
-        dim3 grid(blocks_for(len, 256), (unsigned)((blocks + per_split - 1) / per_split));
-        k_sum_partials<<<grid, 256, 0, st>>>(partial, (int32_t)blocks, len, per_split, counts);
-        le = hipGetLastError();
-    }
-    if (rc == FRMC_OK && le != hipSuccess) {
-        set_error("cell-list histogram launch failed: %s", hipGetErrorString(le));
-        rc = FRMC_EHIP;
-    }
-    (void)hipFreeAsync(scr, st);
     return rc;
 }
 
@@ -949,25 +554,9 @@ static int tune_full(const float *coords, int32_t n, const Basis &B, int isPBC, 
                 // a schedule with fewer items than CUs leaves the chip idle
                 if (full_sched(n, nt, R, 1).items < ncu) continue;
                 bool dup = false;
-                for (const FullChoice &D : cand) dup |= !D.cells && D.nt == nt && D.R == R && D.per_cu == pc;
+                for (const FullChoice &D : cand) dup |= D.nt == nt && D.R == R && D.per_cu == pc;
                 if (!dup) cand.push_back(C);
             }
-    }
-    // the cell-list kernel, when the cell is large enough against the range
-    int32_t mg[3];
-    if (isPBC && cell_grid(B, range_of(A, E), mg)) {
-        const int32_t cnts[2] = {256, 512};
-        for (int32_t nt : cnts) {
-            const int32_t pmax = max_per_cu(lds_bytes + 4 * (size_t)nt, lds, nt);
-            for (int32_t pc = pmax; pc <= 2 * pmax && pc <= kMaxPerCu; pc *= 2) {
-                FullChoice C;
-                C.nt = nt;
-                C.R = 1024 / nt;
-                C.per_cu = pc;
-                C.cells = true;
-                cand.push_back(C);
-            }
-        }
     }
     const int64_t len = 2 * A.size + 4;
     int32_t *scratch = nullptr;
@@ -1050,57 +639,100 @@ static int choose_full(const float *coords, int32_t n, const Basis &B, int isPBC
     return FRMC_OK;
 }
 
-static int launch_full_timed(const float *coords, int32_t n, const Basis &B, int isPBC, bool ortho,
-                             const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E,
-                             int32_t *counts, hipStream_t st);
+// Whether a call takes the chunk pass (full_chunks.hip): every call whose ids,
+// elements and bin offsets fit its packed words, down to the smallest (13
+// atoms: 45 us against 140 for the all-pairs kernel, whose call reads the basis
+// back first).  A forced schedule, and the fixed rule with tuning off, keep
+// the all-pairs kernels.
+static bool chunk_route(int32_t n, const HistArgs &A) {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    return !g_forced_on && g_autotune && chunks_take(n, A);
+}
+
+// HIP events around the pass when per-thread timing is on (frmc_set_timing)
+template <typename Pass>
+static int timed_pass(hipStream_t st, Pass pass) {
+    if (!timing_enabled()) return pass();
+    hipEvent_t a = nullptr, b = nullptr;
+    FRMC_CHECK_HIP(hipEventCreate(&a));
+    FRMC_CHECK_HIP(hipEventCreate(&b));
+    FRMC_CHECK_HIP(hipEventRecord(a, st));
+    int rc = pass();
+    float ms = 0.f;
+    hipError_t e = hipEventRecord(b, st);
+    if (e == hipSuccess) e = hipEventSynchronize(b);
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms, a, b);
+    (void)hipEventDestroy(a);
+    (void)hipEventDestroy(b);
+    if (e != hipSuccess && rc == FRMC_OK) {
+        set_error("kernel timing failed: %s", hipGetErrorString(e));
+        rc = FRMC_EHIP;
+    }
+    set_last_kernel_ms(ms);
+    return rc;
+}
+
+static void device_cus(int &dev, int &ncu) {
+    dev = 0;
+    ncu = 256;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+}
+
+// The chunk pass with its outputs in R, the basis from dbasis or hB.
+static int full_by_chunks(ChunkRun R, const float *coords, int32_t n, const float *dbasis, const Basis &hB, int isPBC,
+                          const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E,
+                          hipStream_t st) {
+    int dev, ncu;
+    device_cus(dev, ncu);
+    int64_t blocks = 0;
+    int32_t nt = 0;
+    R.blocks = &blocks;
+    R.used_nt = &nt;
+    R.pairs = &g_chunks_evaluated;
+    g_chunks_evaluated = -1;
+    const int rc = timed_pass(st, [&] { return run_chunks(R, coords, n, dbasis, hB, isPBC, mol, elem, A, E, ncu, st); });
+    g_last = FullChoice();
+    g_last.nt = nt;
+    g_last.R = 1;  // one row atom per thread
+    g_last_blocks = blocks;
+    g_last_tuned = 1;
+    g_last_evaluated = g_chunks_evaluated;
+    return rc;
+}
 
 // All unordered pairs into counts ([2][nel][nel][H] + overflow, already
 // zeroed or holding counts to add to).  Workgroups count into LDS-private
-// bins and write them to per-workgroup partials, which k_sum_partials adds
+// bins and write them to per-workgroup partials, which add_partials adds
 // into counts (no contention on the global bins); histograms too large for
 // LDS count straight into global memory with atomics.
-int launch_full(const float *coords, int32_t n, const Basis &B, int isPBC, bool ortho, const int32_t *mol,
-                const int32_t *elem, const HistArgs &A, int32_t *counts, hipStream_t st) {
-    return launch_full_timed(coords, n, B, isPBC, ortho, mol, elem, A, nullptr, counts, st);
-}
-
 static int launch_full_timed(const float *coords, int32_t n, const Basis &B, int isPBC, bool ortho,
                              const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E,
                              int32_t *counts, hipStream_t st) {
     if (n < 2) return FRMC_OK;
-    int dev = 0, ncu = 256;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    if (chunk_route(n, A)) {
+        ChunkRun R;
+        R.counts = counts;
+        return full_by_chunks(R, coords, n, nullptr, B, isPBC, mol, elem, A, E, st);
+    }
+    int dev, ncu;
+    device_cus(dev, ncu);
     FullChoice C;
     int tuned = 0;
     if (int rc = choose_full(coords, n, B, isPBC, ortho, mol, elem, A, E, dev, ncu, st, C, tuned)) return rc;
-    hipEvent_t a = nullptr, b = nullptr;
-    const bool timing = timing_enabled();
-    if (timing) {
-        FRMC_CHECK_HIP(hipEventCreate(&a));
-        FRMC_CHECK_HIP(hipEventCreate(&b));
-        FRMC_CHECK_HIP(hipEventRecord(a, st));
-    }
     int64_t blocks = 0;
-    int rc = run_full(C, coords, n, B, isPBC, ortho, mol, elem, A, E, ncu, counts, st, &blocks);
-    if (timing) {
-        float ms = 0.f;
-        hipError_t e = hipEventRecord(b, st);
-        if (e == hipSuccess) e = hipEventSynchronize(b);
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, a, b);
-        (void)hipEventDestroy(a);
-        (void)hipEventDestroy(b);
-        if (e != hipSuccess && rc == FRMC_OK) {
-            set_error("kernel timing failed: %s", hipGetErrorString(e));
-            rc = FRMC_EHIP;
-        }
-        set_last_kernel_ms(ms);
-    }
+    const int rc = timed_pass(
+        st, [&] { return run_full(C, coords, n, B, isPBC, ortho, mol, elem, A, E, ncu, counts, st, &blocks); });
     g_last = C;
     g_last_blocks = blocks;
     g_last_tuned = tuned;
-    g_last_evaluated = C.cells ? g_cells_evaluated : (int64_t)n * (n - 1) / 2;
+    g_last_evaluated = C.cells ? g_chunks_evaluated : (int64_t)n * (n - 1) / 2;
     return rc;
+}
+
+int launch_full(const float *coords, int32_t n, const Basis &B, int isPBC, bool ortho, const int32_t *mol,
+                const int32_t *elem, const HistArgs &A, int32_t *counts, hipStream_t st) {
+    return launch_full_timed(coords, n, B, isPBC, ortho, mol, elem, A, nullptr, counts, st);
 }
 
 // largest |x| of n floats, as the bit pattern of a non-negative float (NaN
@@ -1111,7 +743,23 @@ __global__ void __launch_bounds__(256) k_absmax(const float *__restrict__ x, int
         const float a = fabsf(x[i]);
         m = (a != a) ? __int_as_float(0x7f800000) : fmaxf(m, a);
     }
-    atomicMax(out, __float_as_uint(m));
+    // one atomic per wave (one per lane: 16.4 us at 40,000 atoms)
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(out, __float_as_uint(m));
+}
+
+__global__ void k_copy_words(const uint32_t *__restrict__ from, int n, uint32_t *to) {
+    if ((int)threadIdx.x < n) to[threadIdx.x] = from[threadIdx.x];
+}
+
+// the basis (9 floats) and the largest magnitude's bits to host words; clears the latter
+__global__ void k_edge_inputs(const float *__restrict__ basis, uint32_t *amax, uint32_t *to) {
+    const int t = threadIdx.x;
+    if (t < 9 && basis) to[t] = __float_as_uint(basis[t]);
+    if (t == 9) {
+        to[9] = load_dev(amax);
+        *amax = 0;
+    }
 }
 
 }  // namespace frmc
@@ -1151,12 +799,9 @@ int frmc_multiple_pairs_histograms_coords(const int32_t *indexes, int32_t nidx, 
     FRMC_REQUIRE(nidx == 0 || indexes, "indexes is NULL");
     FRMC_REQUIRE(!isPBC || basis, "basis is NULL");
     hipStream_t st = as_stream(stream);
-    bool ortho = false;
-    Basis hB;
-    if ((rc = read_basis(basis, isPBC, st, hB, ortho))) return rc;
     Scratch sc;
     if ((rc = alloc_counts(sc, A.size, st))) return rc;
-    if ((rc = launch_multi(indexes, nidx, coords, n, basis, isPBC, mol, elem, A, allAtoms, sc.p, st, ortho)))
+    if ((rc = launch_multi(indexes, nidx, coords, n, basis, isPBC, mol, elem, A, allAtoms, sc.p, st)))
         return rc;
     return finish_counts(sc, A.size, hintra, hinter, /*add=*/0, st);
 }
@@ -1196,6 +841,23 @@ int frmc_full_pairs_histograms_coords(const float *coords, int32_t n, const floa
     hipStream_t st = as_stream(stream);
     bool ortho = false;
     Basis hB;
+    if (n >= 2 && chunk_route(n, A)) {
+        HostWords ov(st);
+        if (!ov.p) {
+            set_error("allocation of pinned host words failed");
+            return FRMC_ENOMEM;
+        }
+        ChunkRun R;
+        R.hintra = hintra;
+        R.hinter = hinter;
+        R.overflow = ov.p;
+        memset(&hB, 0, sizeof(hB));
+        if ((rc = full_by_chunks(R, coords, n, isPBC ? basis : nullptr, hB, isPBC, mol, elem, A, nullptr, st)))
+            return rc;
+        FRMC_CHECK_HIP(ov.wait());
+        set_overflow(ov.p[0]);
+        return FRMC_OK;
+    }
     if ((rc = read_basis(basis, isPBC, st, hB, ortho))) return rc;
     Scratch sc;
     if ((rc = alloc_counts(sc, A.size, st))) return rc;
@@ -1260,9 +922,15 @@ int frmc_full_pairs_counts(const float *coords, int32_t n, const float *basis, i
     hipStream_t st = as_stream(stream);
     bool ortho = false;
     Basis hB;
-    if ((rc = read_basis(basis, isPBC, st, hB, ortho))) return rc;
-    k_fill_i32<<<1024, 256, 0, st>>>(counts, 2 * A.size + 1, 0);
+    memset(&hB, 0, sizeof(hB));
+    k_fill_i32<<<std::min(1024u, blocks_for(2 * A.size + 1, 256)), 256, 0, st>>>(counts, 2 * A.size + 1, 0);
     FRMC_CHECK_LAUNCH();
+    if (n >= 2 && chunk_route(n, A)) {
+        ChunkRun R;
+        R.counts = counts;
+        return full_by_chunks(R, coords, n, isPBC ? basis : nullptr, hB, isPBC, mol, elem, A, nullptr, st);
+    }
+    if ((rc = read_basis(basis, isPBC, st, hB, ortho))) return rc;
     return launch_full(coords, n, hB, isPBC, ortho, mol, elem, A, counts, st);
 }
 
@@ -1276,35 +944,36 @@ int frmc_full_pairs_counts_f64(const float *coords, int32_t n, const float *basi
     FRMC_REQUIRE(n == 0 || (coords && mol && elem), "NULL pointer argument");
     FRMC_REQUIRE(!isPBC || basis, "basis is NULL");
     hipStream_t st = as_stream(stream);
-    bool ortho = false;
+    // the basis and the largest coordinate magnitude (which bounds the float32
+    // difference error) reach the host in one wait
+    k_fill_i32<<<std::min(1024u, blocks_for(2 * A.size + 4, 256)), 256, 0, st>>>(counts, 2 * A.size + 4, 0);
+    FRMC_CHECK_LAUNCH();
     Basis hB;
-    if ((rc = read_basis(basis, isPBC, st, hB, ortho))) return rc;
-    // largest coordinate magnitude bounds the float32 difference error
+    memset(&hB, 0, sizeof(hB));
     float amax = 0.0f;
     if (n > 0) {
-        uint32_t *d_m = nullptr;
-        hipError_t e = pool_malloc((void **)&d_m, sizeof(uint32_t), st);
-        if (e != hipSuccess) {
-            set_error("hipMallocAsync failed: %s", hipGetErrorString(e));
+        HostWords in(st);
+        if (!in.p) {
+            set_error("allocation of pinned host words failed");
             return FRMC_ENOMEM;
         }
-        k_fill_i32<<<1, 64, 0, st>>>((int32_t *)d_m, 1, 0);
-        k_absmax<<<256, 256, 0, st>>>(coords, 3 * (int64_t)n, d_m);
-        uint32_t bits = 0;
-        e = hipMemcpyAsync(&bits, d_m, sizeof(bits), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        (void)hipFreeAsync(d_m, st);
-        if (e != hipSuccess) {
-            set_error("coordinate range reduction failed: %s", hipGetErrorString(e));
-            return FRMC_EHIP;
-        }
-        memcpy(&amax, &bits, sizeof(amax));
+        uint32_t *d_m = (uint32_t *)(counts + 2 * A.size + 1);  // not used by the counting
+        k_absmax<<<std::min(64u, blocks_for(3 * (int64_t)n, 256)), 256, 0, st>>>(coords, 3 * (int64_t)n, d_m);
+        k_edge_inputs<<<1, 64, 0, st>>>(isPBC ? basis : nullptr, d_m, (uint32_t *)in.p);
+        FRMC_CHECK_LAUNCH();
+        FRMC_CHECK_HIP(in.wait());
+        const uint32_t *w = (const uint32_t *)in.p;
+        memcpy(&amax, w + 9, sizeof(amax));
+        if (isPBC) memcpy(hB.b, w, sizeof(hB.b));
         FRMC_REQUIRE(amax < 1e30f, "coordinates are not finite");
     }
+    const float *hb = hB.b;
+    const bool ortho = isPBC && hb[1] == 0.f && hb[2] == 0.f && hb[3] == 0.f && hb[5] == 0.f && hb[6] == 0.f && hb[7] == 0.f;
     Edge64 E;
     E.mn = minD;
     E.mx = maxD;
     E.bn = bin;
+    E.amax = amax;
     double rows = 0.0;
     for (int m = 0; m < 3; m++) {
         E.rowsum[m] = isPBC ? fabsf(hB.b[3 * m]) + fabsf(hB.b[3 * m + 1]) + fabsf(hB.b[3 * m + 2]) : 1.0f;
@@ -1315,13 +984,18 @@ int frmc_full_pairs_counts_f64(const float *coords, int32_t n, const float *basi
     const double lo = (double)minD - big, hi = (double)maxD + big;
     E.s_lo = lo > 0.0 ? nextafterf((float)(lo * lo), 0.0f) : 0.0f;
     E.s_hi = nextafterf((float)(hi * hi), INFINITY);
-    k_fill_i32<<<1024, 256, 0, st>>>(counts, 2 * A.size + 4, 0);
-    FRMC_CHECK_LAUNCH();
     rc = launch_full_timed(coords, n, hB, isPBC, ortho, mol, elem, A, &E, counts, st);
     if (rc) return rc;
     if (rechecked) {
-        FRMC_CHECK_HIP(hipMemcpyAsync(rechecked, counts + 2 * A.size + 2, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-        FRMC_CHECK_HIP(hipStreamSynchronize(st));
+        HostWords out(st);
+        if (!out.p) {
+            set_error("allocation of pinned host words failed");
+            return FRMC_ENOMEM;
+        }
+        k_copy_words<<<1, 64, 0, st>>>((const uint32_t *)(counts + 2 * A.size + 2), 2, (uint32_t *)out.p);
+        FRMC_CHECK_LAUNCH();
+        FRMC_CHECK_HIP(out.wait());
+        *rechecked = out.p[0];
     }
     return FRMC_OK;
 }

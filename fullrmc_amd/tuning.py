@@ -2,16 +2,18 @@
 ``frmc_set_autotune``, ``frmc_force_full_schedule``,
 ``frmc_last_full_schedule``).
 
-A schedule of the all-pairs histogram kernel is (threads per workgroup,
-which is also the column tile; row atoms per thread; workgroups per CU).
-Row atoms -1 selects the cell-list kernel (256 or 512 threads), which
-evaluates only pairs in neighbouring cells of a grid at least the
-histogram range wide; it exists for periodic cells with three or more such
-cells per axis (125 or more in all).
-Every schedule gives the same counts, so tuning changes only the time.  With
-tuning on (the default), the first all-pairs call of a shape class times each
-candidate schedule with HIP events and later calls of the class reuse the
-fastest.  The reference has no counterpart: its all-pairs loop
+With tuning on (the default) every call takes the chunk-pruned kernel, whose
+workgroup size follows a rule, unless its inputs do not fit that kernel's packed
+words (more than 64 elements, 2^25 atoms or 2^27 bins).  Those calls, and every
+call with tuning off, evaluate all pairs.  A schedule of the all-pairs
+histogram kernel is (threads per workgroup, which is also the column tile; row
+atoms per thread; workgroups per CU).  With tuning on, the first all-pairs call
+of a shape class times each candidate with HIP events and later calls of the
+class reuse the fastest.  A forced schedule with row atoms -1 (256 or 512
+threads) pins the chunk-pruned kernel's workgroups; it is taken for periodic
+cells with three or more cells of the histogram range per axis (125 or more in
+all).  Every schedule gives the same counts, so tuning changes only the time.
+The reference has no counterpart: its all-pairs loop
 (Extensions/pairs_histograms.pyx:86-176) is one fixed OpenMP loop.
 """
 import ctypes
@@ -38,7 +40,8 @@ def force_full_schedule(threads=None, rowAtoms=None, workgroupsPerCU=None):
 
 
 def last_full_schedule():
-    """The schedule of this thread's last all-pairs call."""
+    """The schedule of this thread's last full-histogram call (the chunk-pruned
+    kernel by rule: one row atom per thread, ``tuned``)."""
     t, r, tuned = ctypes.c_int32(0), ctypes.c_int32(0), ctypes.c_int32(0)
     w = ctypes.c_int64(0)
     _lib.check(_lib.lib().frmc_last_full_schedule(ctypes.byref(t), ctypes.byref(r), ctypes.byref(w),

@@ -49,27 +49,29 @@ float frmc_last_kernel_ms(void);
 
 /* Full-histogram schedule autotuner.  No counterpart in the reference (its
    pairs_histograms.pyx:86-176 has one fixed OpenMP loop); every schedule
-   gives the same counts.  A schedule is (threads per workgroup = column
-   tile: 256, 512 or 1024; row atoms per thread: 1, 2 or 4, or -1 for the
-   cell-list kernel with 256 or 512 threads, available when a periodic cell
-   holds at least three cells of the range's width per axis and 125 in all;
-   workgroups per CU: 1..16, more than fit at once allowed).  With tuning on (the
-   default) the first all-pairs call of a shape class (device, floor(log2 n),
-   bins, boundary kind, float64-recompute mode) times each candidate twice
-   with HIP events on the call's stream, outside the frmc_set_timing window,
-   and later calls of the class reuse the fastest.
-   The tuning call synchronises its stream, so the first call of a class
-   cannot be captured in a HIP graph (tune first, or force a schedule).
+   gives the same counts.  With tuning on (the default) a call takes the
+   chunk-pruned kernel, its workgroup size by a rule, unless it has more than
+   64 elements, 2^25 atoms or 2^27 bins.  Other calls, and every call with
+   tuning off, evaluate all pairs; an all-pairs schedule is (threads per
+   workgroup = column tile: 256, 512 or 1024; row atoms per thread: 1, 2 or 4;
+   workgroups per CU: 1..16, more than fit at once allowed).  Row atoms -1
+   forces the chunk-pruned kernel with 256 or 512 threads, when a periodic
+   cell holds at least three cells of the range's width per axis and 125 in
+   all.  With tuning on, the first all-pairs call of a shape class (device,
+   floor(log2 n), bins, boundary kind, float64-recompute mode) times each
+   candidate twice with HIP events on the call's stream, outside the
+   frmc_set_timing window, and later calls of the class reuse the fastest; that
+   first call synchronises its stream, so it cannot be captured in a HIP graph.
    frmc_set_autotune: 1 on, 0 off (fixed rule), -1 off and forget the
    tuned classes.  frmc_force_full_schedule pins one schedule for every call
    (rowAtoms == 0 releases it).  frmc_last_full_schedule reports the
-   schedule of this thread's last all-pairs call (tuned = 1 when it came
-   from the tuner). */
+   schedule of this thread's last full-histogram call (tuned = 1 when it came
+   from the tuner or the chunk-pruned kernel's rule, whose row atoms are 1). */
 void frmc_set_autotune(int enable);
 int frmc_force_full_schedule(int32_t threads, int32_t rowAtoms, int32_t workgroupsPerCU);
 int frmc_last_full_schedule(int32_t *threads, int32_t *rowAtoms, int64_t *workgroups, int32_t *tuned);
-/* Pairs the last all-pairs call of this thread evaluated: N(N-1)/2, or for
-   the cell-list kernel the pairs in visited cell pairs (counted only while
+/* Pairs the last full-histogram call of this thread evaluated: N(N-1)/2, or
+   for the chunk-pruned kernel those past its tests (counted only while
    frmc_set_timing is on; -1 otherwise).  Measurement only. */
 int frmc_last_full_evaluated(int64_t *pairs);
 

@@ -1,0 +1,99 @@
+"""The chunk-pruned full histogram (full_chunks.hip) against the oracle's
+all-pairs loops: partly filled chunks and columns, odd and even chunk
+numbers, cubic, triclinic and flat cells, open boundaries, coordinates in other
+images, bins in LDS, in global memory and past the end of the array, and the
+binary64 recompute with its count of re-checked pairs."""
+import numpy as np
+import pytest
+
+from fullrmc_amd import systems, tuning
+from fullrmc_amd.Core import pairs_histograms as gph
+from oracle import refcpu
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+CELLS = {"cubic": systems.cubic_basis(31.0), "triclinic": systems.triclinic_basis(30.0, 33.0, 36.0, 70.0, 100.0, 115.0),
+         "flat": systems.triclinic_basis(60.0, 55.0, 9.0, 90.0, 80.0, 95.0), "open": None}
+# nel, min, max, bin, H
+GRIDS = {"lds": (2, 0.0, 9.0, 0.03, 300), "shifted": (3, 1.5, 6.0, 0.05, 90), "inter_lds": (3, 0.0, 8.0, 0.004, 2000),
+         "global": (3, 0.0, 8.0, 0.0005, 16000), "past_end": (2, 0.0, 9.0, 0.03, 200), "wide": (1, 0.0, 40.0, 0.05, 800)}
+
+
+def box(n, cell, seed, images):
+    rng = np.random.default_rng(seed)
+    f = rng.random((n, 3))
+    basis = CELLS[cell] if CELLS[cell] is not None else systems.cubic_basis(31.0)
+    if cell == "open":
+        coords = (f * 31.0 - 7.0).astype(F32)
+    else:
+        coords = (f + (rng.integers(-3, 4, f.shape) if images else 0)).astype(F32)
+    # a fifth of the atoms on a lattice: equal coordinates, half-cell differences
+    coords[: n // 5] = (rng.integers(0, 8, (n // 5, 3)) / 8 * (31.0 if cell == "open" else 1.0)).astype(F32)
+    return coords, basis, (rng.integers(0, max(1, n // 6), n)).astype(np.int32), rng
+
+
+def check(n, cell, grid, images=False, f64=False, seed=0):
+    nel, mn, mx, dr, H = GRIDS[grid]
+    coords, basis, mol, rng = box(n, cell, seed + n, images)
+    elem = rng.integers(0, nel, n).astype(np.int32)
+    args = (coords, basis, cell != "open", mol, elem, nel, F32(mn), F32(mx), F32(dr), H)
+    if f64:
+        ri, re_, rechecked = refcpu.full_pairs_counts_f64(*args, ncores=8)
+        gi, ge, _ = gph.full_pairs_histograms_coords_float64(*args)
+        assert np.array_equal(gi, ri.astype(F32)) and np.array_equal(ge, re_.astype(F32))
+    else:
+        ri, re_ = refcpu.full_pairs_histograms_coords(*args, ncores=8)
+        gi, ge = gph.full_pairs_histograms_coords(*args)
+        assert gi.tobytes() == ri.tobytes() and ge.tobytes() == re_.tobytes()
+    return gi.sum() + ge.sum()
+
+
+@pytest.mark.parametrize("cell", sorted(CELLS))
+@pytest.mark.parametrize("n", [95, 192, 577, 1409, 4096, 4097, 9001])
+def test_sizes_and_cells(n, cell):
+    assert check(n, cell, "lds") > 0
+    assert check(n, cell, "shifted", images=True) > 0
+
+
+@pytest.mark.parametrize("n", [2, 3, 13, 63, 64, 65, 128])
+def test_smallest(n):
+    for cell in sorted(CELLS):
+        check(n, cell, "wide", images=cell != "open", seed=40)
+        check(n, cell, "wide", f64=True, seed=41)
+
+
+@pytest.mark.parametrize("grid", sorted(GRIDS))
+@pytest.mark.parametrize("cell", ["cubic", "triclinic", "open"])
+def test_grids(grid, cell):
+    assert check(2000, cell, grid, seed=5) > 0
+
+
+@pytest.mark.parametrize("cell", sorted(CELLS))
+@pytest.mark.parametrize("grid", ["lds", "shifted", "inter_lds", "wide"])
+def test_binary64(grid, cell):
+    assert check(1500, cell, grid, images=cell != "open", f64=True, seed=9) > 0
+
+
+def test_all_pairs_and_chunks_give_the_same_recheck_count():
+    coords, basis, mol, rng = box(3000, "triclinic", 3, True)
+    elem = rng.integers(0, 2, 3000).astype(np.int32)
+    args = (coords, basis, True, mol, elem, 2, F32(0.0), F32(9.0), F32(0.01), 900)
+    a = gph.full_pairs_histograms_coords_float64(*args)
+    tuning.force_full_schedule(256, 2, 2)
+    try:
+        b = gph.full_pairs_histograms_coords_float64(*args)
+    finally:
+        tuning.force_full_schedule()
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]) and a[2] == b[2] > 0
+
+
+def test_coordinates_that_are_not_finite_are_never_in_range():
+    coords, basis, mol, rng = box(900, "cubic", 4, False)
+    coords[17], coords[400, 1], coords[800, 2] = np.nan, np.inf, -np.inf
+    elem = rng.integers(0, 2, 900).astype(np.int32)
+    grid = (2, F32(0.0), F32(9.0), F32(0.03), 300)
+    got = gph.full_pairs_histograms_coords(coords, basis, True, mol, elem, *grid)
+    keep = np.all(np.isfinite(coords), axis=1)
+    want = refcpu.full_pairs_histograms_coords(coords[keep], basis, True, mol[keep], elem[keep], *grid, ncores=8)
+    assert got[0].tobytes() == want[0].tobytes() and got[1].tobytes() == want[1].tobytes()
