@@ -31,39 +31,17 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "chunks.h"
 #include "full_hist.h"
 
 namespace frmc {
 
 namespace {
 
-constexpr int kNZ = 128;            // counting-sort bins along a column
-constexpr int kBox = 4;             // float4 per chunk box
 constexpr int kListPad = 4;         // a list is padded to the unrolled loop's step
 constexpr int kQueue = 128;         // queued pairs per wave: drained from 64 on
 constexpr int kWaveLds = (64 + kListPad) * 32 + kQueue * 4;
 constexpr int32_t kSelfKey = 1 << 30;
-
-// words of the scratch header (zeroed before the sort, then the plan)
-enum { M_AMAX = 0, M_NCHUNK = 1, M_PAIRS = 4, M_LO = 8, M_HI = 11, M_PLAN = 16, M_WORDS = 64 };
-
-// Lower bound of a squared distance from fractional differences known up to
-// half-widths: |b B|^2 = |b L|^2 with B B^T = L L^T (L lower triangular).
-struct ChunkCut {
-    float L00, L10, L11, L20, L21, L22;
-    float rows;           // sum of |B| (periodic), 1 otherwise
-};
-
-// What follows from the cell, computed on the device: the basis is device
-// memory, and reading it back first cost a synchronisation per call (20 us).
-struct ChunkPlan {
-    Basis B;
-    ChunkCut C;
-    int32_t m0, m1;       // columns across the first two axes
-    int32_t ortho;        // the off-diagonal entries are zero
-};
-constexpr int kPlanWords = sizeof(ChunkPlan) / 4;
-static_assert(sizeof(ChunkPlan) % 4 == 0 && kPlanWords <= 64 && kPlanWords <= M_WORDS - M_PLAN, "plan size");
 
 struct FastBin {
     float inv;            // 1 / bin
@@ -71,12 +49,6 @@ struct FastBin {
     float thi;            // bins below it are inside the range and the row of H bins
     float tie;            // binary64 mode: largest |b| whose image is certain
 };
-
-// Columns across the first two axes, for n atoms: cross-sections of about the
-// side of a cube of 64 atoms, so that 64 consecutive atoms of a column fill
-// about a cube; at most columns_most(n), or the columns' padding outweighs the
-// atoms (flat cells).
-__host__ __device__ __forceinline__ int32_t columns_most(int32_t n) { return n / 96 > 1 ? n / 96 : 1; }
 
 __device__ void make_plan(const float *__restrict__ dbasis, const Basis &hB, int isPBC, int32_t n, ChunkPlan &P) {
     double b[9], h[3] = {1.0, 1.0, 1.0};
@@ -151,19 +123,6 @@ __global__ void __launch_bounds__(256) k_chunk_setup(const float *__restrict__ d
     }
 }
 
-__device__ __forceinline__ uint32_t ordered_bits(float x) {
-    const uint32_t b = __float_as_uint(x);
-    return b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
-}
-__device__ __forceinline__ float from_ordered(uint32_t u) {
-    return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
-}
-
-__device__ __forceinline__ float abs_or_inf(float x) {
-    const float a = fabsf(x);
-    return a == a ? a : __uint_as_float(0x7f800000u);
-}
-
 // open boundaries: the coordinates' extent (maxima of the ordered bits and of their complements)
 __global__ void __launch_bounds__(256) k_chunk_extent(const float *__restrict__ coords, int32_t n,
                                                       uint32_t *__restrict__ meta) {
@@ -228,18 +187,6 @@ __global__ void __launch_bounds__(256) k_chunk_count(const float *__restrict__ c
     a = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
     if (threadIdx.x == 0 && a > 1.0f && __float_as_uint(a) > load_dev(meta + M_AMAX))
         atomicMax(&meta[M_AMAX], __float_as_uint(a));
-}
-
-// the largest |coordinate| (at least 1), infinite if one is not a number
-template <bool PBC>
-__device__ __forceinline__ float coord_max(const uint32_t *__restrict__ meta) {
-    if (PBC) return fmaxf(1.0f, __uint_as_float(load_dev(meta + M_AMAX)));
-    float a = 1.0f;
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-        a = fmaxf(a, fmaxf(abs_or_inf(from_ordered(~load_dev(meta + M_LO + k))),
-                           abs_or_inf(from_ordered(load_dev(meta + M_HI + k)))));
-    return a;
 }
 
 __device__ __forceinline__ int32_t wave_scan(int32_t v, int lane) {
@@ -471,49 +418,6 @@ __global__ void __launch_bounds__(256) k_chunk_boxes(const float4 *__restrict__ 
         b[2] = make_float4(from[0], from[1], from[2], 0.0f);
         b[3] = make_float4(to[0], to[1], to[2], 0.0f);
     }
-}
-
-// x - min_image(x): the image taken, which never falls as x grows
-__device__ __forceinline__ float image_of(float x) { return copysignf(floorf(fabsf(x) + 0.5f), x); }
-
-// Squared lower bound of the distance of any pair whose wrapped differences
-// lie within w of d.  Per row of L: |b_k L_kk| is at least L_kk (|d_k| - w_k)
-// whatever image is taken; where no axis of the row can cross +-1/2, the
-// row's interval is used instead.
-template <bool PBC, bool ORTHO>
-__device__ __forceinline__ float lower_bound2(float d0, float d1, float d2, float w0, float w1, float w2,
-                                              const ChunkCut &C) {
-    if (PBC) {
-        d0 -= rintf(d0);
-        d1 -= rintf(d1);
-        d2 -= rintf(d2);
-    }
-    float x = (fabsf(d0) - w0) * C.L00, y = (fabsf(d1) - w1) * C.L11, z = (fabsf(d2) - w2) * C.L22;
-    if (PBC && !ORTHO) {
-        const float M0 = fabsf(d0) + w0, M1 = fabsf(d1) + w1, M2 = fabsf(d2) + w2;
-        const float a10 = fabsf(C.L10), a20 = fabsf(C.L20), a21 = fabsf(C.L21);
-        const bool s12 = fmaxf(M1, M2) < 0.5f, s012 = fmaxf(M0, fmaxf(M1, M2)) < 0.5f;
-        y -= a21 * fminf(M2, 0.5f);
-        x -= a10 * fminf(M1, 0.5f) + a20 * fminf(M2, 0.5f);
-        const float ys = fabsf(d1 * C.L11 + d2 * C.L21) - (w1 * C.L11 + w2 * a21);
-        const float xs = fabsf(d0 * C.L00 + d1 * C.L10 + d2 * C.L20) - (w0 * C.L00 + w1 * a10 + w2 * a20);
-        y = s12 ? fmaxf(y, ys) : y;
-        x = s012 ? fmaxf(x, xs) : x;
-    }
-    x = fmaxf(x, 0.0f);
-    y = fmaxf(y, 0.0f);
-    z = fmaxf(z, 0.0f);
-    return x * x + y * y + z * z;
-}
-
-// The range with a margin for every rounding between the bound above and the
-// float32 distance: differences of coordinates up to amax (2^-24 each, times
-// sum |B|), the image, the product with the basis, norm and sqrt (1e-5).
-// Squared; infinite when a coordinate is not finite (then nothing is skipped).
-__device__ __forceinline__ float cut_squared(const ChunkCut &C, float range, float amax) {
-    const float w = range * 1.00001f + C.rows * 9.5367431640625e-07f * (amax + 1.0f);
-    const float w2 = w * w * 1.00001f;
-    return w2 == w2 ? w2 : __uint_as_float(0x7f800000u);
 }
 
 struct ChunkArgs {
@@ -789,16 +693,10 @@ __device__ __forceinline__ void full_chunks(const ChunkArgs &K, const Basis &B, 
     }
 }
 
-// The plan reaches every wave through one lane-varying load and broadcasts
-// (see load_dev); orthorhombic cells take their shorter arithmetic.
+// Orthorhombic cells take their shorter arithmetic.
 template <bool PBC, bool LDS_HIST, bool EDGE>
 __global__ void __launch_bounds__(1024, EDGE ? 4 : 8) k_full_chunks(ChunkArgs K, Edge64 E) {
-    const uint32_t v = K.meta[M_PLAN + min((int)(threadIdx.x & 63), kPlanWords - 1)];
-    uint32_t w[kPlanWords];
-#pragma unroll
-    for (int k = 0; k < kPlanWords; k++) w[k] = (uint32_t)__builtin_amdgcn_readlane((int)v, k);
-    ChunkPlan P;
-    __builtin_memcpy(&P, w, sizeof(P));
+    const ChunkPlan P = plan_of(K.meta);
     if (PBC && P.ortho)
         full_chunks<PBC, true, LDS_HIST, EDGE>(K, P.B, P.C, E);
     else
@@ -874,6 +772,64 @@ FastBin fast_bin(const HistArgs &A, const Edge64 *E, int isPBC) {
 
 }  // namespace
 
+ChunkSort chunk_layout(int32_t n) {
+    ChunkSort S;
+    memset(&S, 0, sizeof(S));
+    S.ncol = columns_most(n);
+    S.cells = S.ncol * kNZ;
+    S.maxchunks = (n + 63) / 64 + S.ncol;
+    const size_t np = (size_t)S.maxchunks * 64;
+    size_t off = 4 * M_WORDS;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off = (off + bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    S.o_cnt = take(4 * (size_t)S.cells);
+    S.o_start = take(4 * (size_t)S.cells);
+    S.o_tot = take(4 * (size_t)S.ncol);
+    S.o_base = take(4 * (size_t)S.ncol);
+    S.o_where = take(8 * (size_t)n);
+    S.o_sx = take(16 * np);
+    S.o_mol = take(4 * np);
+    S.o_box = take(sizeof(float4) * kBox * (size_t)S.maxchunks);
+    S.bytes = off;
+    return S;
+}
+
+void launch_chunk_sort(ChunkSort &S, char *scr, const float *coords, int32_t n, const float *dbasis, const Basis &hB,
+                       int isPBC, const int32_t *mol, const int32_t *elem, int32_t nel, int32_t *zero, int64_t nzero,
+                       hipStream_t st) {
+    uint32_t *meta = S.meta = (uint32_t *)scr;
+    float4 *sx = S.sx = (float4 *)(scr + S.o_sx), *cbox = S.cbox = (float4 *)(scr + S.o_box);
+    int32_t *smol = S.smol = (int32_t *)(scr + S.o_mol);
+    int32_t *cnt = (int32_t *)(scr + S.o_cnt), *start = (int32_t *)(scr + S.o_start), *tot = (int32_t *)(scr + S.o_tot),
+            *base = (int32_t *)(scr + S.o_base);
+    int2 *where = (int2 *)(scr + S.o_where);
+    const unsigned nb = blocks_for(n, 256), cb = (unsigned)((S.maxchunks + 3) / 4);
+    if (n <= kSmallSort && isPBC) {
+        k_chunk_sort_small<true><<<1, 1024, 0, st>>>(dbasis, hB, coords, n, mol, elem, nel, meta, where, sx, smol, zero,
+                                                     nzero);
+    } else if (n <= kSmallSort) {
+        k_chunk_sort_small<false><<<1, 1024, 0, st>>>(dbasis, hB, coords, n, mol, elem, nel, meta, where, sx, smol, zero,
+                                                      nzero);
+    } else {
+        k_chunk_setup<<<std::min(512u, blocks_for(S.cells + nzero, 256)), 256, 0, st>>>(dbasis, hB, isPBC, n, meta, cnt,
+                                                                                        S.cells, zero, nzero);
+        if (!isPBC) k_chunk_extent<<<std::min(nb, 64u), 256, 0, st>>>(coords, n, meta);
+        if (isPBC)
+            k_chunk_count<true><<<nb, 256, 0, st>>>(coords, n, meta, cnt, where);
+        else
+            k_chunk_count<false><<<nb, 256, 0, st>>>(coords, n, meta, cnt, where);
+        k_chunk_scan<<<1, 1024, 0, st>>>((const int2 *)cnt, (int2 *)start, tot, base, meta, sx, smol);
+        k_chunk_scatter<<<nb, 256, 0, st>>>(coords, n, mol, elem, nel, where, start, base, sx, smol);
+    }
+    if (isPBC)
+        k_chunk_boxes<true><<<cb, 256, 0, st>>>(sx, meta, cbox);
+    else
+        k_chunk_boxes<false><<<cb, 256, 0, st>>>(sx, meta, cbox);
+}
+
 bool chunks_take(int32_t n, const HistArgs &A) { return A.nel <= 64 && n < (1 << 25) && A.size < (1 << 27); }
 
 int add_partials(const int32_t *partial, int64_t nparts, int64_t size, int32_t *counts, hipStream_t st) {
@@ -885,7 +841,8 @@ int add_partials(const int32_t *partial, int64_t nparts, int64_t size, int32_t *
 
 int run_chunks(const ChunkRun &R, const float *coords, int32_t n, const float *dbasis, const Basis &hB, int isPBC,
                const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E, int ncu, hipStream_t st) {
-    const int64_t ncol = columns_most(n), cells = ncol * kNZ, maxchunks = (n + 63) / 64 + ncol;
+    ChunkSort S = chunk_layout(n);
+    const int64_t maxchunks = S.maxchunks;
     // bins in LDS: both halves, else the inter-molecular half, else none
     const size_t kMaxHist = 112 * 1024;  // leaves eight waves' lists of the 160 KB
     const int64_t size = A.size;
@@ -926,59 +883,24 @@ int run_chunks(const ChunkRun &R, const float *coords, int32_t n, const float *d
     if (R.blocks) *R.blocks = blocks;
     if (R.used_nt) *R.used_nt = nt;
 
-    const size_t np = (size_t)maxchunks * 64;
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        const size_t at = off;
-        off = (off + bytes + 255) & ~(size_t)255;
-        return at;
-    };
     const int64_t ncounts = R.counts ? 0 : 2 * size + 4;
-    const size_t o_meta = take(4 * M_WORDS), o_cnt = take(4 * (size_t)cells), o_counts = take(4 * (size_t)ncounts),
-                 o_start = take(4 * (size_t)cells), o_tot = take(4 * (size_t)ncol), o_base = take(4 * (size_t)ncol),
-                 o_where = take(8 * (size_t)n), o_sx = take(16 * np), o_mol = take(4 * np),
-                 o_box = take(sizeof(float4) * kBox * (size_t)maxchunks), o_part = take(hist_bytes * (size_t)blocks);
+    const size_t o_counts = S.bytes, o_part = (o_counts + 4 * (size_t)ncounts + 255) & ~(size_t)255,
+                 bytes = o_part + hist_bytes * (size_t)blocks;
     char *scr = nullptr;
-    hipError_t e = pool_malloc((void **)&scr, off, st);
+    hipError_t e = pool_malloc((void **)&scr, bytes, st);
     if (e != hipSuccess) {
-        set_error("hipMallocAsync of %zu bytes for the full histogram failed: %s", off, hipGetErrorString(e));
+        set_error("hipMallocAsync of %zu bytes for the full histogram failed: %s", bytes, hipGetErrorString(e));
         return FRMC_ENOMEM;
     }
-    uint32_t *meta = (uint32_t *)(scr + o_meta);
-    int32_t *cnt = (int32_t *)(scr + o_cnt), *start = (int32_t *)(scr + o_start), *tot = (int32_t *)(scr + o_tot),
-            *base = (int32_t *)(scr + o_base), *smol = (int32_t *)(scr + o_mol),
-            *counts = R.counts ? R.counts : (int32_t *)(scr + o_counts);
-    int2 *where = (int2 *)(scr + o_where);
-    float4 *sx = (float4 *)(scr + o_sx), *cbox = (float4 *)(scr + o_box);
-    const unsigned nb = blocks_for(n, 256), cb = (unsigned)((maxchunks + 3) / 4);
-    if (n <= kSmallSort && isPBC) {
-        k_chunk_sort_small<true><<<1, 1024, 0, st>>>(dbasis, hB, coords, n, mol, elem, A.nel, meta, where, sx, smol, counts,
-                                                     ncounts);
-    } else if (n <= kSmallSort) {
-        k_chunk_sort_small<false><<<1, 1024, 0, st>>>(dbasis, hB, coords, n, mol, elem, A.nel, meta, where, sx, smol, counts,
-                                                      ncounts);
-    } else {
-        k_chunk_setup<<<std::min(512u, blocks_for(cells + ncounts, 256)), 256, 0, st>>>(dbasis, hB, isPBC, n, meta, cnt,
-                                                                                        cells, counts, ncounts);
-        if (!isPBC) k_chunk_extent<<<std::min(nb, 64u), 256, 0, st>>>(coords, n, meta);
-        if (isPBC)
-            k_chunk_count<true><<<nb, 256, 0, st>>>(coords, n, meta, cnt, where);
-        else
-            k_chunk_count<false><<<nb, 256, 0, st>>>(coords, n, meta, cnt, where);
-        k_chunk_scan<<<1, 1024, 0, st>>>((const int2 *)cnt, (int2 *)start, tot, base, meta, sx, smol);
-        k_chunk_scatter<<<nb, 256, 0, st>>>(coords, n, mol, elem, A.nel, where, start, base, sx, smol);
-    }
-    if (isPBC)
-        k_chunk_boxes<true><<<cb, 256, 0, st>>>(sx, meta, cbox);
-    else
-        k_chunk_boxes<false><<<cb, 256, 0, st>>>(sx, meta, cbox);
+    int32_t *counts = R.counts ? R.counts : (int32_t *)(scr + o_counts);
+    launch_chunk_sort(S, scr, coords, n, dbasis, hB, isPBC, mol, elem, A.nel, counts, ncounts, st);
     Edge64 none;
     memset(&none, 0, sizeof(none));
     const Edge64 &EE = E ? *E : none;
-    K.sx = sx;
-    K.smol = smol;
-    K.cbox = cbox;
-    K.meta = meta;
+    K.sx = S.sx;
+    K.smol = S.smol;
+    K.cbox = S.cbox;
+    K.meta = S.meta;
     K.range = E ? (float)sqrt((double)E->s_hi) : A.g.maxD;
     K.A = A;
     K.F = fast_bin(A, E, isPBC);
@@ -1013,7 +935,7 @@ int run_chunks(const ChunkRun &R, const float *coords, int32_t n, const float *d
             R.counts ? nullptr : R.hinter, R.overflow);
     e = hipGetLastError();
     if (e == hipSuccess && K.count_pairs) {
-        e = hipMemcpyAsync(R.pairs, meta + M_PAIRS, sizeof(int64_t), hipMemcpyDeviceToHost, st);
+        e = hipMemcpyAsync(R.pairs, S.meta + M_PAIRS, sizeof(int64_t), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
     }
     (void)hipFreeAsync(scr, st);

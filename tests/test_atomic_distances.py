@@ -7,6 +7,7 @@ import itertools
 import numpy as np
 import pytest
 
+from fullrmc_amd import systems
 from fullrmc_amd.Core import atomic_distances as gad
 from oracle import refcpu
 
@@ -250,3 +251,36 @@ def test_many_counted_pairs_13500_atoms():
     ref = refcpu.full_atomic_distances_coords(box, s["basis"], True, mol, elem, 2, lo, up, flags)
     assert sum(int(x.sum()) for x in (got[0], got[2])) > 1_000_000
     assert _same(got, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cell", ["cubic", "triclinic", "open"])
+@pytest.mark.parametrize("limit", [0.4, 1.6, 3.5])
+def test_near_pairs_of_many_atoms_match_oracle(cell, limit):
+    """6,001 atoms, enough pairs for the chunk-pruned pass: no, few and more
+    selected pairs than one workgroup sorts; the whole system, and a list with
+    repeated atoms against all atoms and against the later ones."""
+    rng = np.random.default_rng(17)
+    n, nel = 6001, 3
+    basis = (systems.triclinic_basis(42.0, 44.0, 46.0, 80.0, 95.0, 105.0) if cell == "triclinic"
+             else systems.cubic_basis(43.0))
+    box = (rng.random((n, 3)) + rng.integers(-1, 2, (n, 3))).astype(F32)
+    coords = (rng.random((n, 3)) * 43.0).astype(F32) if cell == "open" else box
+    coords[:50] = coords[50:100]  # distances of exactly zero
+    mol = rng.integers(0, 900, n).astype(np.int32)
+    elem = rng.integers(0, nel, n).astype(np.int32)
+    lo, up = _limits(nel, 0.0, limit, seed=5)
+    kw = dict(interMolecular=True, intraMolecular=True, countWithinLimits=True, reduceDistanceToUpper=True)
+    flags = refcpu.ad_flags(True, True, True, True)
+    pbc = cell != "open"
+    got = gad.full_atomic_distances_coords(coords, basis, pbc, mol, elem, nel, lo, up, **kw)
+    ref = refcpu.full_atomic_distances_coords(coords, basis, pbc, mol, elem, nel, lo, up, flags)
+    assert got[0].sum() + got[2].sum() > 0
+    assert _same(got, ref)
+    idx = rng.integers(0, n, 6000).astype(np.int32)
+    for allAtoms in (True, False):
+        got = gad.multiple_atomic_distances_coords(idx, coords, basis, pbc, mol, elem, nel, lo, up, allAtoms=allAtoms,
+                                                   **kw)
+        ref = refcpu.multiple_atomic_distances_coords(idx, coords, basis, pbc, mol, elem, nel, lo, up, flags,
+                                                      allAtoms=allAtoms)
+        assert _same(got, ref)
