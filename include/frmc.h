@@ -294,11 +294,9 @@ int frmc_sq_transform(const float *Gr, int32_t k, int32_t H, const float *sqMatr
 /* frmc_sq_transform without any allocation.  No counterpart in the
    reference: it is for callers that cannot allocate device memory (code
    under HIP graph capture, allocation-free serving loops).  Same arguments
-   and results (bit-identical in both modes); the matrix-core mode keeps its
-   split partials in a library-owned device array of at most 2^22 floats
-   (16 MiB) per GPU, held until the process ends, and returns FRMC_EINVAL
-   when a shape needs more.  All calls on one GPU share that array: calls
-   that overlap on one GPU race. */
+   and results (bit-identical in both modes).  The matrix-core mode returns
+   FRMC_EINVAL for shapes whose r range, split over about 1,024 output tiles
+   of 64 x 64, would give more than 2^22 partial floats. */
 int frmc_sq_transform_noalloc(const float *Gr, int32_t k, int32_t H, const float *sqMatrix, int32_t nQ,
                               int addOne, int mode, float *Sq, void *stream);
 

@@ -161,3 +161,24 @@ def test_sq_to_Gr_vs_oracle():
     got = grs.sq_to_Gr(q, rv, S)
     ref = orc.sq_to_Gr(q, rv, S)
     assert _ulps(got, ref).max() <= 1 or np.max(np.abs(got - ref)) < 1e-6 * np.max(np.abs(ref))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [1, 15, 63, 64, 65, 130, 200])
+@pytest.mark.parametrize("k,nQ", [(1, 1), (3, 64), (5, 65), (33, 17), (2100, 3), (4101, 2)])
+def test_sq_transform_edges_of_tiles(k, H, nQ):
+    """Partly filled chunks of rows, tiles of Q and groups of curves (one, two and
+    four per wave): the exact mode is the sequential sum bit for bit, the matrix cores
+    stay within float32 rounding of the terms' magnitudes."""
+    rng = np.random.default_rng(k + H + nQ)
+    G = rng.standard_normal((k, H)).astype(F32)
+    M = rng.standard_normal((H, nQ)).astype(F32)
+    S = grs.sq_transform(G, M, addOne=False)
+    ref = np.zeros((k, nQ), F32)
+    for r in range(H):  # NumPy's axis-0 order (its sum of a single column would be pairwise)
+        ref += G[:, r:r + 1] * M[r]
+    assert S.tobytes() == ref.tobytes()
+    T = grs.sq_transform(G, M, addOne=False, mode="mfma").astype(np.float64)
+    exact, terms = G.astype(np.float64) @ M.astype(np.float64), np.abs(G).astype(np.float64) @ np.abs(M)
+    # at most H roundings of 2^-24 relative to the sum of magnitudes, plus the products'
+    assert np.all(np.abs(T - exact) <= (H + 1) * 2.0 ** -24 * terms)
