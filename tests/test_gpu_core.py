@@ -256,3 +256,25 @@ def test_full_histogram_float64_recompute_40000_atoms():
     ci, ce, ov = refcpu.full_pairs_counts_f64(*args, ncores=8)
     assert same(gi, ci.astype(F32)) and same(ge, ce.astype(F32))
     assert 0 < rechecked < 0.05 * (gi.sum() + ge.sum())
+
+
+@pytest.mark.parametrize("isPBC", [True, False])
+@pytest.mark.parametrize("n,k", [(1, 1), (255, 3), (257, 16), (300, 255), (300, 256), (290, 257), (33, 600)])
+def test_tiles_of_points_and_atoms(sysm, isPBC, n, k):
+    """Distances and differences of k points to n atoms around the tiles' edges,
+    from every atom on and from all."""
+    rng = np.random.default_rng(n + k)
+    coords = np.ascontiguousarray((sysm["box"] if isPBC else sysm["real"])[:n])
+    idx = rng.integers(0, n, k).astype(np.int32)
+    pts = rng.standard_normal((3, k)).astype(F32)
+    B = sysm["basis"]
+    assert same(gpd.pairs_distances_to_multi_indexcoords(idx, coords, B, isPBC),
+                refcpu.pairs_distances_to_multi_indexcoords(idx, coords, B, isPBC))
+    assert same(gpd.pairs_distances_to_multi_points(pts, coords, B, isPBC),
+                refcpu.pairs_distances_to_multi_points(pts, coords, B, isPBC))
+    assert same(gpd.pairs_differences_to_multi_indexcoords(idx, coords, B, isPBC),
+                refcpu.pairs_differences_to_multi_indexcoords(idx, coords, B, isPBC))
+    got = gpd.pairs_distances_to_multi_indexcoords(idx, coords, B, isPBC, allAtoms=False)
+    ref = refcpu.pairs_distances_to_multi_indexcoords(idx, coords, B, isPBC)
+    later = np.arange(n)[:, None] >= idx[None, :]
+    assert same(got[later], ref[later])
