@@ -87,6 +87,7 @@ struct View {
     int32_t Hmax, Mmax, maxLeaves, nunits;
     // window
     const int32_t *pgroup, *poff;  // staging (host-mapped)
+    int32_t gmaxw;                 // most atoms a proposal of the window moves
     const int32_t *patoms;         // the moved atoms per proposal (at poff), or null: the group's
     const float *pold, *pnew;
     int32_t *dn;                   // delta buffer of this window
@@ -264,6 +265,18 @@ struct CommitCtl {
 // workload (k_delta 17.3 us; 2: 17.5, 4: 18.7) -- more blocks, fewer
 // proposals' atomics per thread
 constexpr int kDP = 1;
+// Windows of groups (k_delta_groups, k_commit on a group): threads of a
+// block, dealt over up to kGroupParts of the group's atoms and as many other
+// atoms as that leaves; the most blocks of a launch (more work goes to each
+// instead of zeroing and flushing more copies of the bins: 13-atom groups,
+// k = 16, 52,000 atoms, 1,000 bins: 46.2 us a window with 512 blocks, 46.3 with
+// 256, 48.0 with 1,024, 53 with a block per tile); a block's LDS at most (two
+// blocks per compute unit; at 128 KB windows of 2-atom groups with 1,000 bins
+// took 32.8 us against 28.3).
+constexpr int kGroupThreads = 1024;  // a 13-atom window of 6,500 atoms: 35.9 us, at 512 38.2, at 256 48.6
+constexpr int kGroupParts = 8;
+constexpr int32_t kGroupBlocks = 512;
+constexpr int32_t kGroupLds = 80 * 1024;
 
 // Windows of many engines (replicas) launched together, one launch per kernel
 // (single-atom moves).  The views are uploaded once per run; each step

@@ -50,6 +50,7 @@ View make_view(frmc_engine *e, int s) {
     V.nunits = e->nunits;
     V.pgroup = e->stage[s].d_pgroup;
     V.poff = e->stage[s].d_poff;
+    V.gmaxw = e->stage[s].lists ? e->lcap : e->gmax;
     V.patoms = e->stage[s].lists ? e->stage[s].d_patoms : nullptr;
     V.pold = e->stage[s].d_pold;
     V.pnew = e->stage[s].d_pnew;

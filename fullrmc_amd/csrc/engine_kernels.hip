@@ -133,6 +133,85 @@ __device__ __forceinline__ void commit_pair(const View &V, float s, int32_t ea, 
     }
 }
 
+// ints of all constraints' slots
+__host__ __device__ __forceinline__ int32_t slot_ints(const View &V) {
+    int64_t n = 0;
+    for (int32_t ci = 0; ci < V.C; ci++) n += 2ll * V.nel * V.nel * V.c[ci].H;
+    return (int32_t)(n < (1ll << 30) ? n : 1ll << 30);
+}
+
+// commit_pair on a copy of the slots in LDS, the constraints' one after another
+__device__ __forceinline__ void commit_pair_lds(const View &V, int32_t *bins, float s, int32_t ea, int32_t eb,
+                                                bool intra, int32_t sign) {
+    int32_t b = -1, at = 0;
+    for (int32_t ci = 0; ci < V.C; ci++) {
+        const DevC &c = V.c[ci];
+        const int32_t size = V.nel * V.nel * c.H;
+        if (!c.sameGrid) b = in_range(s, c.g) ? bin_of(s, c.g) : -1;
+        if (b >= 0) {
+            const int32_t f = flat_slot(b, ea, eb, V.nel, c.H);
+            if (f >= 0) atomicAdd(&bins[at + (intra ? 0 : size) + f], sign);
+            else if (sign > 0) atomicAdd(&c.slot[2 * size], 1);  // past the array: counted, not stored
+        }
+        at += 2 * size;
+    }
+}
+
+// Pairs in range of some constraint, gathered by a wave: the range test takes
+// a few operations, the bin a square root and a divide, and in a large box
+// most lanes fail the test.  A lane queues its pair when the old or the new
+// distance is in range, and 64 queued pairs are binned by a full wave.
+struct HitQueue {
+    float o[128], w[128];
+    int32_t tag[128];  // below 64 before a push
+};
+
+struct HitRange {
+    float lo, hi;
+    __device__ bool hit(float so, float sn) const { return (so >= lo && so < hi) || (sn >= lo && sn < hi); }
+};
+
+__device__ __forceinline__ HitRange hit_range(const View &V) {
+    HitRange R = {V.c[0].g.s_lo, V.c[0].g.s_hi};
+    for (int32_t ci = 1; ci < V.C; ci++) {
+        R.lo = fminf(R.lo, V.c[ci].g.s_lo);
+        R.hi = fmaxf(R.hi, V.c[ci].g.s_hi);
+    }
+    return R;
+}
+
+// all lanes of the wave call it; bin(so, sn, tag) takes 64 pairs at a time
+template <class Bin>
+__device__ __forceinline__ void push_hits(HitQueue &Q, int32_t &len, bool hit, float so, float sn, int32_t tag,
+                                          const Bin &bin) {
+    const uint64_t m = __ballot(hit);
+    if (!m) return;
+    if (hit) {
+        const int32_t at = len + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        Q.o[at] = so;
+        Q.w[at] = sn;
+        Q.tag[at] = tag;
+    }
+    len += __popcll(m);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (len >= 64) {
+        len -= 64;
+        const int32_t at = len + (threadIdx.x & 63);
+        bin(Q.o[at], Q.w[at], Q.tag[at]);
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <class Bin>
+__device__ __forceinline__ void flush_hits(const HitQueue &Q, int32_t &len, const Bin &bin) {
+    const int32_t at = threadIdx.x & 63;
+    if (at < len) bin(Q.o[at], Q.w[at], Q.tag[at]);
+    len = 0;
+    __builtin_amdgcn_wave_barrier();
+}
+
 // grid (ceil(n/256), ceil(k/kDP)): one other atom per thread, kDP proposals
 // per block; deltas go straight into the proposal's (zeroed) block of dn.
 // P.valid: the previous window's accepted single-atom move is committed here
@@ -265,6 +344,79 @@ __global__ void __launch_bounds__(256) k_delta(View V, Inline I, Pending Parg, i
     const Pending P = pending_of(V, Parg);
     if (PROPS) delta_body<PBC, ORTHO>(V, PropSrc{V.props}, P, V.dn, k, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, G);
     else delta_body<PBC, ORTHO>(V, InlineSrc{I}, P, V.dn, k, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, G);
+}
+
+// group atoms that a block takes side by side, kGroupThreads / parts other atoms each
+__host__ __device__ __forceinline__ int32_t group_parts(int32_t g) {
+    int32_t parts = 1;
+    while (parts < kGroupParts && parts < g) parts *= 2;
+    return parts;
+}
+
+// The pairs of a group in G with the other atoms, dealt over the launch's
+// blocks (blockIdx.x of gridDim.x): bin(so, sn, tag) is called by full waves
+// with 64 pairs in range of some constraint; tag = intra << 12 | ea << 6 | eb.
+template <bool PBC, bool ORTHO, bool MOL, class Bin>
+__device__ __forceinline__ void group_pairs(const View &V, const GroupLds &G, HitQueue &Q, const Bin &bin) {
+    const int32_t lane = threadIdx.x & 63, g = G.g;
+    const int32_t parts = group_parts(g), width = kGroupThreads / parts;  // width: a power of two of at least 64
+    const int32_t id = lane < g ? G.id[lane] : -1;
+    const HitRange R = hit_range(V);
+    int32_t len = 0;
+    for (int32_t j0 = blockIdx.x * width; j0 < V.n; j0 += gridDim.x * width) {
+        const int32_t j = j0 + (threadIdx.x & (width - 1)), jj = min(j, V.n - 1);
+        const float cx = V.xyz[3 * (int64_t)jj], cy = V.xyz[3 * (int64_t)jj + 1], cz = V.xyz[3 * (int64_t)jj + 2];
+        const int32_t ej = V.elem[jj], mj = MOL ? V.mol[jj] : 0;
+        // the group's own atoms among the wave's 64
+        const int32_t at = id - (j - lane);
+        uint64_t in = __ballot(lane < g && at >= 0 && at < 64), own = 0;
+        for (; in; in &= in - 1) own |= 1ull << __builtin_amdgcn_readlane(at, __builtin_ctzll(in));
+        const bool other = j < V.n && !(own >> lane & 1);
+        for (int32_t a = threadIdx.x / width; a < g; a += parts) {
+            const float so = pair_s<PBC, ORTHO>(G.o[a][0], G.o[a][1], G.o[a][2], cx, cy, cz, V.B);
+            const float sn = pair_s<PBC, ORTHO>(G.w[a][0], G.w[a][1], G.w[a][2], cx, cy, cz, V.B);
+            const int32_t intra = MOL && G.mol[a] == mj;
+            push_hits(Q, len, other && R.hit(so, sn), so, sn, intra << 12 | G.el[a] << 6 | ej, bin);
+        }
+    }
+    flush_hits(Q, len, bin);
+}
+
+// Window of groups: the blocks (., p) count proposal p's deltas in LDS, each
+// for its share of the other atoms, and add the bins that changed.  What
+// bound the direct form was its atomics: a window of 16 proposals of 13 atoms
+// among 6,500 made about 450,000, and atomics on one cache line of the delta
+// blocks follow one another at about 30 ns (22 us a launch, 7 with the
+// atomics taken out).  Bins in LDS are added once per block, and 32
+// neighbouring bins of a line in one request: 7.7 us.
+template <bool PBC, bool ORTHO>
+__global__ void __launch_bounds__(kGroupThreads) k_delta_groups(View V) {
+    extern __shared__ int32_t gbins[];  // dnStride
+    __shared__ GroupLds G;
+    __shared__ HitQueue queue[kGroupThreads / 64];
+    const int tid = threadIdx.x;
+    load_group(V, blockIdx.y, G);
+    for (int32_t s = tid; s < V.dnStride; s += kGroupThreads) gbins[s] = 0;
+    __syncthreads();
+    const int32_t g = G.g;
+    group_pairs<PBC, ORTHO, false>(V, G, queue[tid / 64], [&](float so, float sn, int32_t tag) {
+        delta_pair<PBC, ORTHO>(V, gbins, so, sn, tag >> 6, tag & 63);
+    });
+    // group-internal pairs: M - F leaves each unordered pair once, in slot
+    // [e(later position), e(earlier position)]
+    if (blockIdx.x == 0) {
+        for (int32_t q = tid; q < g * (g - 1) / 2; q += kGroupThreads) {
+            int32_t a, b;
+            decode_pair(q, a, b);
+            const float so = pair_s<PBC, ORTHO>(G.o[a][0], G.o[a][1], G.o[a][2], G.o[b][0], G.o[b][1], G.o[b][2], V.B);
+            const float sn = pair_s<PBC, ORTHO>(G.w[a][0], G.w[a][1], G.w[a][2], G.w[b][0], G.w[b][1], G.w[b][2], V.B);
+            delta_pair<PBC, ORTHO>(V, gbins, so, sn, G.el[a], G.el[b]);
+        }
+    }
+    __syncthreads();
+    int32_t *out = V.dn + (int64_t)blockIdx.y * V.dnStride;
+    for (int32_t s = tid; s < V.dnStride; s += kGroupThreads)
+        if (gbins[s]) atomicAdd(&out[s], gbins[s]);
 }
 
 // ------------------------------------------------------- k_delta, chunk walk
@@ -1363,15 +1515,19 @@ __global__ void __launch_bounds__(256) k_eval_b_batch(BatchArgs A) {
 // ---------------------------------------------------------------- k_commit
 
 
-// grid ceil(n/256): picks the proposal to commit (every block makes the same
+// GROUP: a group's pairs, counted in LDS as in k_delta_groups (18.9 us to 9.5
+// in the window described there); else grid ceil(n/256), one other atom per
+// thread.  Picks the proposal to commit (every block makes the same
 // decision from the window's totals), then slot counts of the accepted group
 // vs every other atom (one atom per thread), pair-type sums += the proposal's
 // deltas, and the group's new coordinates (block 0; no block reads the
 // group's coordinates).  The group comes from the kernel arguments (single-atom
 // windows: old coordinates from the host mirror) or the staging buffers.
-template <bool PBC, bool ORTHO>
-__global__ void __launch_bounds__(256) k_commit(View V, Inline I, CommitCtl C) {
+template <bool PBC, bool ORTHO, bool GROUP>
+__global__ void __launch_bounds__(GROUP ? kGroupThreads : 256) k_commit(View V, Inline I, CommitCtl C) {
+    extern __shared__ int32_t sbins[];  // GROUP: the constraints' slots
     __shared__ GroupLds G;
+    __shared__ HitQueue queue[GROUP ? kGroupThreads / 64 : 1];
     const int tid = threadIdx.x;
     int32_t p = C.p;
     if (p < 0) {
@@ -1406,6 +1562,8 @@ __global__ void __launch_bounds__(256) k_commit(View V, Inline I, CommitCtl C) {
     } else {
         load_group(V, p, G);
     }
+    if (GROUP)
+        for (int32_t s = tid; s < slot_ints(V); s += blockDim.x) sbins[s] = 0;
     __syncthreads();
     const int64_t gt = (int64_t)blockIdx.x * blockDim.x + tid, gs = (int64_t)gridDim.x * blockDim.x;
     const int32_t *dn = C.dn + (int64_t)p * V.dnStride;
@@ -1414,19 +1572,36 @@ __global__ void __launch_bounds__(256) k_commit(View V, Inline I, CommitCtl C) {
         for (int64_t s = gt; s < (int64_t)V.T * c.H; s += gs) c.base[s] += dn[c.dnOff + s];
     }
     const int32_t g = G.g;
-    const int32_t j = (int32_t)gt;
-    if (j < V.n) {
-        bool member = false;
-        for (int32_t a = 0; a < g; a++) member |= (G.id[a] == j);
-        if (!member) {
-            const float cx = V.xyz[3 * (int64_t)j], cy = V.xyz[3 * (int64_t)j + 1], cz = V.xyz[3 * (int64_t)j + 2];
-            const int32_t ej = V.elem[j], mj = V.mol[j];
-            for (int32_t a = 0; a < g; a++) {
-                const float so = pair_s<PBC, ORTHO>(G.o[a][0], G.o[a][1], G.o[a][2], cx, cy, cz, V.B);
-                const float sn = pair_s<PBC, ORTHO>(G.w[a][0], G.w[a][1], G.w[a][2], cx, cy, cz, V.B);
-                const bool intra = G.mol[a] == mj;
-                commit_pair<PBC, ORTHO>(V, so, G.el[a], ej, intra, -1);
-                commit_pair<PBC, ORTHO>(V, sn, G.el[a], ej, intra, +1);
+    if (GROUP) {
+        // (coordinates of the group's own atoms, which block 0 writes, are read and not used)
+        group_pairs<PBC, ORTHO, true>(V, G, queue[tid / 64], [&](float so, float sn, int32_t tag) {
+            commit_pair_lds(V, sbins, so, (tag >> 6) & 63, tag & 63, (tag >> 12) != 0, -1);
+            commit_pair_lds(V, sbins, sn, (tag >> 6) & 63, tag & 63, (tag >> 12) != 0, +1);
+        });
+        __syncthreads();
+        int32_t at = 0;
+        for (int32_t ci = 0; ci < V.C; ci++) {
+            const DevC &c = V.c[ci];
+            const int32_t size = 2 * V.nel * V.nel * c.H;
+            for (int32_t s = tid; s < size; s += blockDim.x)
+                if (sbins[at + s]) atomicAdd(&c.slot[s], sbins[at + s]);
+            at += size;
+        }
+    } else {
+        const int32_t j = (int32_t)gt;
+        if (j < V.n) {
+            bool member = false;
+            for (int32_t a = 0; a < g; a++) member |= (G.id[a] == j);
+            if (!member) {
+                const float cx = V.xyz[3 * (int64_t)j], cy = V.xyz[3 * (int64_t)j + 1], cz = V.xyz[3 * (int64_t)j + 2];
+                const int32_t ej = V.elem[j], mj = V.mol[j];
+                for (int32_t a = 0; a < g; a++) {
+                    const float so = pair_s<PBC, ORTHO>(G.o[a][0], G.o[a][1], G.o[a][2], cx, cy, cz, V.B);
+                    const float sn = pair_s<PBC, ORTHO>(G.w[a][0], G.w[a][1], G.w[a][2], cx, cy, cz, V.B);
+                    const bool intra = G.mol[a] == mj;
+                    commit_pair<PBC, ORTHO>(V, so, G.el[a], ej, intra, -1);
+                    commit_pair<PBC, ORTHO>(V, sn, G.el[a], ej, intra, +1);
+                }
             }
         }
     }
@@ -1484,6 +1659,31 @@ __global__ void k_fill(int32_t *__restrict__ p, int64_t n) {
 
 // ------------------------------------------------------------------ launch
 
+// Counting a group's pairs in LDS: the bins fit a block and are not many more
+// than its pairs.  Windows against one atomic per pair (k = 16, 6,500 atoms,
+// 300 bins): 2 atoms 29.5 us against 31.6, 4 atoms 31.2 against 35.7, 9 atoms
+// 32.9 against 46.5; 52,000 atoms and 1,000 bins: 30.4 against 31.3, 34.1
+// against 35.2, 39.9 against 43.7.
+static bool group_bins_fit(const View &V, int64_t ints) {
+    const int64_t fixed = sizeof(GroupLds) + sizeof(HitQueue) * (kGroupThreads / 64);
+    return V.gmaxw > 1 && ints <= 4096ll * V.gmaxw && fixed + 4 * ints <= kGroupLds;
+}
+
+// blocks per proposal of k proposals
+static unsigned group_blocks(const View &V, int32_t k) {
+    const unsigned tiles = blocks_for(V.n, kGroupThreads / group_parts(V.gmaxw));
+    return std::min(tiles, std::max(1u, (unsigned)(kGroupBlocks / k)));
+}
+
+template <bool PBC, bool ORTHO>
+static void launch_k_delta_groups(const View &V, dim3 grid, hipStream_t st) {
+    const size_t shm = sizeof(int32_t) * (size_t)V.dnStride;
+    if (shm > 32 * 1024)
+        (void)hipFuncSetAttribute((const void *)k_delta_groups<PBC, ORTHO>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)shm);
+    k_delta_groups<PBC, ORTHO><<<grid, kGroupThreads, shm, st>>>(V);
+}
+
 int launch_delta(const View &V, const Inline &I, const Pending &P, int32_t k, hipStream_t st) {
     if (V.prune) {
         // single-atom proposals in a periodic box: the chunk walk
@@ -1502,6 +1702,14 @@ int launch_delta(const View &V, const Inline &I, const Pending &P, int32_t k, hi
             else if (src == 1) k_delta_chunks<false, 1><<<grid, 256, 0, st>>>(V, I, P, k, pp);
             else k_delta_chunks<false, 2><<<grid, 256, 0, st>>>(V, I, P, k, pp);
         }
+        FRMC_CHECK_LAUNCH();
+        return FRMC_OK;
+    }
+    if (I.k == 0 && !V.props && !P.valid && group_bins_fit(V, V.dnStride)) {
+        const dim3 ggrid(group_blocks(V, k), (unsigned)k);
+        if (!V.isPBC) launch_k_delta_groups<false, false>(V, ggrid, st);
+        else if (V.ortho) launch_k_delta_groups<true, true>(V, ggrid, st);
+        else launch_k_delta_groups<true, false>(V, ggrid, st);
         FRMC_CHECK_LAUNCH();
         return FRMC_OK;
     }
@@ -1612,14 +1820,26 @@ size_t eval_b_lds_bytes(const View &V) {
     return sizeof(float) * (V.Mmax + V.maxLeaves + kStack + (size_t)2 * V.maxLeaves);
 }
 
+template <bool PBC, bool ORTHO, bool GROUP>
+static void launch_k_commit(const View &V, const Inline &I, const CommitCtl &C, hipStream_t st) {
+    const size_t shm = GROUP ? sizeof(int32_t) * (size_t)slot_ints(V) : 0;
+    if (shm > 32 * 1024)
+        (void)hipFuncSetAttribute((const void *)k_commit<PBC, ORTHO, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)shm);
+    const unsigned blocks = GROUP ? group_blocks(V, 1) : blocks_for(V.n, 256);
+    k_commit<PBC, ORTHO, GROUP><<<blocks, GROUP ? kGroupThreads : 256, shm, st>>>(V, I, C);
+}
+
+template <bool GROUP>
+static void launch_k_commit_cell(const View &V, const Inline &I, const CommitCtl &C, hipStream_t st) {
+    if (!V.isPBC) launch_k_commit<false, false, GROUP>(V, I, C, st);
+    else if (V.ortho) launch_k_commit<true, true, GROUP>(V, I, C, st);
+    else launch_k_commit<true, false, GROUP>(V, I, C, st);
+}
+
 int launch_commit(const View &V, const Inline &I, const CommitCtl &C, hipStream_t st) {
-    const unsigned g = blocks_for(V.n, 256);
-    if (V.isPBC) {
-        if (V.ortho) k_commit<true, true><<<g, 256, 0, st>>>(V, I, C);
-        else k_commit<true, false><<<g, 256, 0, st>>>(V, I, C);
-    } else {
-        k_commit<false, false><<<g, 256, 0, st>>>(V, I, C);
-    }
+    if (I.k == 0 && group_bins_fit(V, slot_ints(V))) launch_k_commit_cell<true>(V, I, C, st);
+    else launch_k_commit_cell<false>(V, I, C, st);
     FRMC_CHECK_LAUNCH();
     return FRMC_OK;
 }

@@ -850,3 +850,36 @@ def test_molecular_triclinic_full_size():
     dlog = []
     E.run_device(40, k=8, log=dlog)
     assert_same_state(E, oe, dlog, olog, (pys, nps))
+
+
+@pytest.mark.parametrize("n,sizes,k,nbins,cell", [
+    (67, (1, 2, 64), 4, 60, "cubic"),            # one wave and a remainder; the largest group
+    (700, (1, 2, 3, 5, 13, 33, 64), 16, 140, "triclinic"),  # ragged groups around the parts of a block
+    (1290, (2,), 7, 140, "cubic"),               # two atoms: 512 other atoms per tile, remainder
+    (1290, (2,), 7, 2800, "triclinic"),          # bins past 4,096 a group atom
+    (700, (9,), 5, 5000, "cubic"),               # bins past the LDS of a block
+    (5003, (13, 40), 64, 140, "cubic"),          # several tiles per block
+])
+def test_group_windows_match_oracle_at_the_edges_of_blocks(n, sizes, k, nbins, cell):
+    """Windows of ragged groups inside larger molecules, two grids: the state
+    after the run equals the oracle's exactly, on both counting paths."""
+    rng = np.random.default_rng(n + nbins)
+    basis = systems.cubic_basis(22.0) if cell == "cubic" else systems.triclinic_basis(22.0, 23.0, 24.0, 80, 95, 105)
+    real = (rng.random((n, 3)) @ basis.astype(np.float64)).astype(F32)
+    s = dict(real=real, elements=[("O", "Si")[i] for i in rng.integers(0, 2, n)],
+             molecules=(np.arange(n) // 70).astype(np.int32), basis=basis, recip=systems.reciprocal(basis))
+    groups, at = [], 0
+    while at < n:
+        g = min(sizes[len(groups) % len(sizes)], n - at)
+        groups.append(list(range(at, at + g)))
+        at += g
+    exps = [pdc_target(s, 0.05, 8, 0.025, 7.0 / nbins, nbins), pdc_target(s, 0.05, 9, 0.4, 0.11, 50)]
+    oe, olog, pys, nps = oracle_run(s, groups, oeng.Translation(0.3),
+                                    lambda osys, w: [oeng.PDC(osys, e, w) for e in exps], 40, 21, tolerance=5.0)
+    random.seed(21)
+    np.random.seed(21)
+    E = device_engine(s, [PairDistributionConstraint(e) for e in exps], groups=groups, gen=TranslationGenerator(0.3))
+    E.set_tolerance(5.0)
+    dlog = []
+    E.run_device(40, k=k, log=dlog)
+    assert_same_state(E, oe, dlog, olog, (pys, nps))
