@@ -382,7 +382,7 @@ static int run_batched(std::vector<TranslationRun> &runs, int32_t T) {
         shm_a = std::max(shm_a, eval_lds_bytes(hv[r]));
         shm_b = std::max(shm_b, eval_b_lds_bytes(hv[r]));
         kmax = std::max(kmax, runs[r].k);
-        maxd += (int64_t)((hv[r].n + kChunk - 1) / kChunk) * ((runs[r].k + kBP - 1) / kBP);
+        maxd += batch_delta_blocks(hv[r].n, runs[r].k);
         maxa += (int64_t)hv[r].nunits * runs[r].k;
     }
     FRMC_REQUIRE(maxd < ((int64_t)1 << 30) && maxa < ((int64_t)1 << 30), "batched grid too large");
@@ -417,7 +417,7 @@ static int run_batched(std::vector<TranslationRun> &runs, int32_t T) {
         const int32_t n = (int32_t)l.reps.size();
         int64_t md = 0, ma = 0;
         for (int32_t r : l.reps) {
-            md += (int64_t)((hv[r].n + kChunk - 1) / kChunk) * ((runs[r].k + kBP - 1) / kBP);
+            md += batch_delta_blocks(hv[r].n, runs[r].k);
             ma += (int64_t)hv[r].nunits * runs[r].k;
         }
         l.win_b = align16(sizeof(BatchWin) * n);
@@ -503,7 +503,7 @@ static int run_batched(std::vector<TranslationRun> &runs, int32_t T) {
         int32_t nd = 0, na = 0, nb = 0;
         for (int32_t i = 0; i < l.nact; i++) {
             const View &V = hv[l.act[i]];
-            const int32_t k = l.kws[i], bd = ((V.n + kChunk - 1) / kChunk) * ((k + kBP - 1) / kBP);
+            const int32_t k = l.kws[i], bd = batch_delta_blocks(V.n, k);
             for (int32_t q = 0; q < bd; q++) hm[nd++] = make_int2(i, q);
         }
         for (int32_t i = 0; i < l.nact; i++) {
@@ -592,7 +592,7 @@ static int run_batched_loop(std::vector<TranslationRun> &runs) {
         shm_b = std::max(shm_b, eval_b_lds_bytes(hv[r]));
         shm_l = std::max(shm_l, sizeof(float) * (size_t)runs[r].k * e->resW);
         kmax = std::max(kmax, runs[r].k);
-        maxd += (int64_t)((hv[r].n + kChunk - 1) / kChunk) * ((runs[r].k + kBP - 1) / kBP);
+        maxd += batch_delta_blocks(hv[r].n, runs[r].k);
         maxa += (int64_t)hv[r].nunits * runs[r].k;
         maxb += runs[r].k;
     }
@@ -709,7 +709,7 @@ static int run_batched_loop(std::vector<TranslationRun> &runs) {
             }
         }
         for (int32_t r = 0; r < R; r++) {
-            const int32_t bd = ((hv[r].n + kChunk - 1) / kChunk) * ((kr[r] + kBP - 1) / kBP);
+            const int32_t bd = batch_delta_blocks(hv[r].n, kr[r]);
             for (int32_t q = 0; q < bd; q++) h_maps[nd++] = make_int2(r, q);
         }
         for (int32_t r = 0; r < R; r++)

@@ -293,6 +293,11 @@ constexpr int32_t kChunk = 2048;
 // when the host bounded a step, 1 was fastest: 3.21M; 2: 3.18M; 4: 2.64M)
 constexpr int32_t kBP = 2;
 constexpr int32_t kBatchLdsInts = 8192;  // largest kBP delta blocks counted in LDS there (32 KB)
+// workgroups of k_delta_batch for a window of k proposals among n atoms: per
+// chunk one for each kBP proposals and one for the pending commit's slots
+inline int32_t batch_delta_blocks(int32_t n, int32_t k) {
+    return ((n + kChunk - 1) / kChunk) * ((k + kBP - 1) / kBP + 1);
+}
 struct BatchWin {
     int32_t rep;             // replica (index into the views)
     int32_t k, prop;         // proposals, first of them in the proposal table

@@ -161,9 +161,10 @@ __device__ __forceinline__ void commit_pair_lds(const View &V, int32_t *bins, fl
 // a few operations, the bin a square root and a divide, and in a large box
 // most lanes fail the test.  A lane queues its pair when the old or the new
 // distance is in range, and 64 queued pairs are binned by a full wave.
+template <int N>
 struct HitQueue {
-    float o[128], w[128];
-    int32_t tag[128];  // below 64 before a push
+    float o[N], w[N];
+    int32_t tag[N];
 };
 
 struct HitRange {
@@ -180,12 +181,10 @@ __device__ __forceinline__ HitRange hit_range(const View &V) {
     return R;
 }
 
-// all lanes of the wave call it; bin(so, sn, tag) takes 64 pairs at a time
-template <class Bin>
-__device__ __forceinline__ void push_hits(HitQueue &Q, int32_t &len, bool hit, float so, float sn, int32_t tag,
-                                          const Bin &bin) {
+// all lanes of the wave call it
+template <int N>
+__device__ __forceinline__ void push_hits(HitQueue<N> &Q, int32_t &len, bool hit, float so, float sn, int32_t tag) {
     const uint64_t m = __ballot(hit);
-    if (!m) return;
     if (hit) {
         const int32_t at = len + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
@@ -194,18 +193,26 @@ __device__ __forceinline__ void push_hits(HitQueue &Q, int32_t &len, bool hit, f
         Q.tag[at] = tag;
     }
     len += __popcll(m);
+}
+
+// bin(so, sn, tag) on 64 queued pairs at a time, until fewer are left
+template <int N, class Bin>
+__device__ __forceinline__ void drain_hits(const HitQueue<N> &Q, int32_t &len, const Bin &bin) {
+    if (len < 64) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    if (len >= 64) {
+    while (len >= 64) {
         len -= 64;
         const int32_t at = len + (threadIdx.x & 63);
         bin(Q.o[at], Q.w[at], Q.tag[at]);
-        __builtin_amdgcn_wave_barrier();
     }
+    __builtin_amdgcn_wave_barrier();
 }
 
-template <class Bin>
-__device__ __forceinline__ void flush_hits(const HitQueue &Q, int32_t &len, const Bin &bin) {
+template <int N, class Bin>
+__device__ __forceinline__ void flush_hits(const HitQueue<N> &Q, int32_t &len, const Bin &bin) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     const int32_t at = threadIdx.x & 63;
     if (at < len) bin(Q.o[at], Q.w[at], Q.tag[at]);
     len = 0;
@@ -357,7 +364,7 @@ __host__ __device__ __forceinline__ int32_t group_parts(int32_t g) {
 // blocks (blockIdx.x of gridDim.x): bin(so, sn, tag) is called by full waves
 // with 64 pairs in range of some constraint; tag = intra << 12 | ea << 6 | eb.
 template <bool PBC, bool ORTHO, bool MOL, class Bin>
-__device__ __forceinline__ void group_pairs(const View &V, const GroupLds &G, HitQueue &Q, const Bin &bin) {
+__device__ __forceinline__ void group_pairs(const View &V, const GroupLds &G, HitQueue<128> &Q, const Bin &bin) {
     const int32_t lane = threadIdx.x & 63, g = G.g;
     const int32_t parts = group_parts(g), width = kGroupThreads / parts;  // width: a power of two of at least 64
     const int32_t id = lane < g ? G.id[lane] : -1;
@@ -376,7 +383,8 @@ __device__ __forceinline__ void group_pairs(const View &V, const GroupLds &G, Hi
             const float so = pair_s<PBC, ORTHO>(G.o[a][0], G.o[a][1], G.o[a][2], cx, cy, cz, V.B);
             const float sn = pair_s<PBC, ORTHO>(G.w[a][0], G.w[a][1], G.w[a][2], cx, cy, cz, V.B);
             const int32_t intra = MOL && G.mol[a] == mj;
-            push_hits(Q, len, other && R.hit(so, sn), so, sn, intra << 12 | G.el[a] << 6 | ej, bin);
+            push_hits(Q, len, other && R.hit(so, sn), so, sn, intra << 12 | G.el[a] << 6 | ej);
+            drain_hits(Q, len, bin);
         }
     }
     flush_hits(Q, len, bin);
@@ -393,7 +401,7 @@ template <bool PBC, bool ORTHO>
 __global__ void __launch_bounds__(kGroupThreads) k_delta_groups(View V) {
     extern __shared__ int32_t gbins[];  // dnStride
     __shared__ GroupLds G;
-    __shared__ HitQueue queue[kGroupThreads / 64];
+    __shared__ HitQueue<128> queue[kGroupThreads / 64];
     const int tid = threadIdx.x;
     load_group(V, blockIdx.y, G);
     for (int32_t s = tid; s < V.dnStride; s += kGroupThreads) gbins[s] = 0;
@@ -1360,6 +1368,16 @@ __device__ __forceinline__ void commit_pair_x(const DeltaCtx &X, float s, int32_
     }
 }
 
+__device__ __forceinline__ HitRange hit_range_x(const DeltaCtx &X) {
+    HitRange R = {X.g[0].s_lo, X.g[0].s_hi};
+#pragma unroll
+    for (int ci = 1; ci < kMaxC; ci++) {
+        R.lo = fminf(R.lo, X.g[ci].s_lo);  // past C: a copy of the first
+        R.hi = fmaxf(R.hi, X.g[ci].s_hi);
+    }
+    return R;
+}
+
 // One workgroup per (group pb of up to kBP proposals, chunk ch of kChunk
 // other atoms) of a replica's window: each other atom's coordinates are read
 // once for the group's proposals, whose pair-type deltas are counted in LDS
@@ -1367,17 +1385,23 @@ __device__ __forceinline__ void commit_pair_x(const DeltaCtx &X, float s, int32_
 // when one chunk covers all atoms (the workgroup owns the blocks), else added
 // bin by bin -- or, without LDSB, added straight to the (zeroed) blocks.  The
 // replica's pending commit is spread over its workgroups as in k_delta:
-// pair-type sums (grid-stride), slot counts (the pb == 0 workgroups, each for
-// its chunk), the moved atom's coordinates (one thread).
+// pair-type sums (grid-stride), the moved atom's coordinates (one thread);
+// its slot counts are one more workgroup's per chunk.
+// 48 replicas of 1,000 to 20,000 atoms, 4 proposals each: 24.1 us a launch
+// with every wave binning its own few pairs in range and the slot counts made
+// by the first group's workgroups; 18.9 with the pairs queued for full waves;
+// 14.4 with the slot counts apart and the next atom loaded ahead (4.7 of it
+// before and after the loop).
 template <bool PBC, bool ORTHO, bool LDSB>
 __device__ __forceinline__ void delta_chunk(const View &V, const BatchWin &W, const Prop *props, int32_t pb,
-                                            int32_t ch, int32_t nch, int32_t *bins) {
+                                            int32_t ch, int32_t nch, int32_t *bins,
+                                                HitQueue<64 * (kBP + 1)> &Q) {
     // props: this workgroup's kBP proposals (staged in LDS), props[q] for q < np
     const int tid = threadIdx.x;
     DeltaCtx X;
     load_ctx(V, X);
     const int32_t dnStride = V.dnStride, T = V.T, k = W.k;
-    const int32_t p0 = pb * kBP, np = min(kBP, k - p0);
+    const int32_t p0 = pb * kBP, np = max(0, min(kBP, k - p0));
     int32_t *out = W.dn + (int64_t)p0 * dnStride;
     const Pending P = pending_of(V, W.P);  // (device window loop: the replica's loop state)
     int32_t qa[kBP], qe[kBP];
@@ -1400,7 +1424,8 @@ __device__ __forceinline__ void delta_chunk(const View &V, const BatchWin &W, co
     }
     int32_t *acc = LDSB ? bins : out;
     const bool pv = P.valid != 0;
-    const int32_t nblk = ((k + kBP - 1) / kBP) * nch;
+    const int32_t npb = (k + kBP - 1) / kBP;
+    const int32_t nblk = (npb + 1) * nch;
     if (pv) {
         const int64_t gt = ((int64_t)pb * nch + ch) * blockDim.x + tid;
         const int64_t gs = (int64_t)nblk * blockDim.x;
@@ -1412,35 +1437,61 @@ __device__ __forceinline__ void delta_chunk(const View &V, const BatchWin &W, co
         if (pb == 0 && ch == 0 && tid == 0)
             for (int d = 0; d < 3; d++) V.xyz[3 * (int64_t)P.atom + d] = P.nw[d];
     }
-    const int32_t pmol = pv ? X.mol[P.atom] : 0;
-    const int32_t j1 = min(X.n, (ch + 1) * kChunk);
-#pragma unroll 2
-    for (int32_t j = ch * kChunk + tid; j < j1; j += blockDim.x) {
-        float cx = X.xyz[3 * (int64_t)j], cy = X.xyz[3 * (int64_t)j + 1], cz = X.xyz[3 * (int64_t)j + 2];
-        const int32_t ej = X.elem[j];
-        if (pv) {
-            if (pb == 0 && j != P.atom) {
-                const float so = pair_s<PBC, ORTHO>(P.old[0], P.old[1], P.old[2], cx, cy, cz, X.B);
-                const float sn = pair_s<PBC, ORTHO>(P.nw[0], P.nw[1], P.nw[2], cx, cy, cz, X.B);
-                const bool intra = pmol == X.mol[j];
-                commit_pair_x(X, so, P.el, ej, intra, -1);
-                commit_pair_x(X, sn, P.el, ej, intra, +1);
-            }
-            if (j == P.atom) {
-                cx = P.nw[0];
-                cy = P.nw[1];
-                cz = P.nw[2];
-            }
+    const int32_t j0 = ch * kChunk, j1 = min(X.n, j0 + kChunk);
+    const HitRange R = hit_range_x(X);
+    // the thread's other atom of the chunk's 256 from jb on; each is loaded
+    // while the one before it is worked on
+    struct Other {
+        float x, y, z;
+        int32_t el;
+    };
+    auto other = [&](int32_t jb) {
+        const int32_t jj = min(jb + tid, j1 - 1);
+        return Other{X.xyz[3 * (int64_t)jj], X.xyz[3 * (int64_t)jj + 1], X.xyz[3 * (int64_t)jj + 2], X.elem[jj]};
+    };
+    int32_t len = 0;
+    if (pb == npb) {
+        // the pending commit's slot counts over this chunk
+        if (!pv) return;
+        const int32_t pmol = X.mol[P.atom];
+        auto bin = [&](float so, float sn, int32_t tag) {
+            commit_pair_x(X, so, P.el, tag & 63, (tag >> 6) != 0, -1);
+            commit_pair_x(X, sn, P.el, tag & 63, (tag >> 6) != 0, +1);
+        };
+        Other o = other(j0), next;
+        int32_t mol = X.mol[min(j0 + tid, j1 - 1)], nextmol;
+        for (int32_t jb = j0; jb < j1; jb += blockDim.x, o = next, mol = nextmol) {
+            next = other(jb + blockDim.x);
+            nextmol = X.mol[min(jb + (int32_t)blockDim.x + tid, j1 - 1)];
+            const int32_t j = jb + tid;
+            const float so = pair_s<PBC, ORTHO>(P.old[0], P.old[1], P.old[2], o.x, o.y, o.z, X.B);
+            const float sn = pair_s<PBC, ORTHO>(P.nw[0], P.nw[1], P.nw[2], o.x, o.y, o.z, X.B);
+            push_hits(Q, len, j < j1 && j != P.atom && R.hit(so, sn), so, sn, (pmol == mol) << 6 | o.el);
+            drain_hits(Q, len, bin);
         }
+        flush_hits(Q, len, bin);
+        return;
+    }
+    auto bin = [&](float so, float sn, int32_t tag) {
+        delta_pair_x(X, acc + (tag >> 12) * dnStride, so, sn, (tag >> 6) & 63, tag & 63);
+    };
+    Other o = other(j0), next;
+    for (int32_t jb = j0; jb < j1; jb += blockDim.x, o = next) {
+        next = other(jb + blockDim.x);
+        const int32_t j = jb + tid;
+        const bool moved = pv && j == P.atom;
+        const float cx = moved ? P.nw[0] : o.x, cy = moved ? P.nw[1] : o.y, cz = moved ? P.nw[2] : o.z;
 #pragma unroll
         for (int q = 0; q < kBP; q++) {
-            if (q >= np || j == qa[q]) continue;
+            if (q >= np) continue;
             // M counts (moved atom a, other j) with diff = c[a] - c[j], before and after
             const float so = pair_s<PBC, ORTHO>(ox[q], oy[q], oz[q], cx, cy, cz, X.B);
             const float sn = pair_s<PBC, ORTHO>(nx[q], ny[q], nz[q], cx, cy, cz, X.B);
-            delta_pair_x(X, acc + q * dnStride, so, sn, qe[q], ej);
+            push_hits(Q, len, j < j1 && j != qa[q] && R.hit(so, sn), so, sn, q << 12 | qe[q] << 6 | o.el);
         }
+        drain_hits(Q, len, bin);
     }
+    flush_hits(Q, len, bin);
     if (LDSB) {
         __syncthreads();
         if (nch == 1) {
@@ -1454,20 +1505,19 @@ __device__ __forceinline__ void delta_chunk(const View &V, const BatchWin &W, co
 
 template <bool PBC, bool ORTHO>
 __device__ __forceinline__ void delta_chunk_any(const View &V, const BatchWin &W, const Prop *props, int32_t pb,
-                                                int32_t ch, int32_t nch, int32_t *bins) {
-    if (kBP * V.dnStride <= kBatchLdsInts) delta_chunk<PBC, ORTHO, true>(V, W, props, pb, ch, nch, bins);
-    else delta_chunk<PBC, ORTHO, false>(V, W, props, pb, ch, nch, bins);
+                                                int32_t ch, int32_t nch, int32_t *bins,
+                                                HitQueue<64 * (kBP + 1)> &Q) {
+    if (kBP * V.dnStride <= kBatchLdsInts) delta_chunk<PBC, ORTHO, true>(V, W, props, pb, ch, nch, bins, Q);
+    else delta_chunk<PBC, ORTHO, false>(V, W, props, pb, ch, nch, bins, Q);
 }
 
-// at most 128 VGPRs (four waves per SIMD): the unconstrained 130 allowed
-// three, and 256 replicas ran 8 % faster with four (3.57M against 3.30M
-// moves/s; five waves need a register spill).  With two proposals per
-// workgroup the bound spills 57 VGPRs to scratch and still wins: 5.41M
-// against 4.99M moves/s with three waves and no spill.
+// at most 128 VGPRs (four waves per SIMD): 256 replicas ran 8 % faster with
+// four than with three.  109 are used.
 __global__ void __launch_bounds__(256, 4) k_delta_batch(BatchArgs A) {
     extern __shared__ int32_t bins[];  // kBP delta blocks (the largest that fits kBatchLdsInts)
     __shared__ BatchLds S;
     __shared__ Prop sp[kBP];
+    __shared__ HitQueue<64 * (kBP + 1)> queue[4];
     stage_block(S, A.map_d, A);
     const BatchWin &W = S.W;
     const View &V = S.V;
@@ -1475,7 +1525,7 @@ __global__ void __launch_bounds__(256, 4) k_delta_batch(BatchArgs A) {
     const int32_t pb = S.m.y / nch, ch = S.m.y % nch;
     {
         // the workgroup's proposals (those past the window's end are not read)
-        const int32_t p0 = pb * kBP, np = min(kBP, W.k - p0);
+        const int32_t p0 = pb * kBP, np = min(kBP, W.k - p0);  // none for the commit's
         const uint32_t *src = reinterpret_cast<const uint32_t *>(A.props + W.prop + p0);
         uint32_t *dst = reinterpret_cast<uint32_t *>(sp);
         for (int i = threadIdx.x; i < np * (int)(sizeof(Prop) / 4); i += blockDim.x) dst[i] = load_dev(src + i);
@@ -1483,10 +1533,10 @@ __global__ void __launch_bounds__(256, 4) k_delta_batch(BatchArgs A) {
     }
     const Prop *props = sp;
     if (V.isPBC) {
-        if (V.ortho) delta_chunk_any<true, true>(V, W, props, pb, ch, nch, bins);
-        else delta_chunk_any<true, false>(V, W, props, pb, ch, nch, bins);
+        if (V.ortho) delta_chunk_any<true, true>(V, W, props, pb, ch, nch, bins, queue[threadIdx.x / 64]);
+        else delta_chunk_any<true, false>(V, W, props, pb, ch, nch, bins, queue[threadIdx.x / 64]);
     } else {
-        delta_chunk_any<false, false>(V, W, props, pb, ch, nch, bins);
+        delta_chunk_any<false, false>(V, W, props, pb, ch, nch, bins, queue[threadIdx.x / 64]);
     }
 }
 
@@ -1527,7 +1577,7 @@ template <bool PBC, bool ORTHO, bool GROUP>
 __global__ void __launch_bounds__(GROUP ? kGroupThreads : 256) k_commit(View V, Inline I, CommitCtl C) {
     extern __shared__ int32_t sbins[];  // GROUP: the constraints' slots
     __shared__ GroupLds G;
-    __shared__ HitQueue queue[GROUP ? kGroupThreads / 64 : 1];
+    __shared__ HitQueue<128> queue[GROUP ? kGroupThreads / 64 : 1];
     const int tid = threadIdx.x;
     int32_t p = C.p;
     if (p < 0) {
@@ -1665,7 +1715,7 @@ __global__ void k_fill(int32_t *__restrict__ p, int64_t n) {
 // 32.9 against 46.5; 52,000 atoms and 1,000 bins: 30.4 against 31.3, 34.1
 // against 35.2, 39.9 against 43.7.
 static bool group_bins_fit(const View &V, int64_t ints) {
-    const int64_t fixed = sizeof(GroupLds) + sizeof(HitQueue) * (kGroupThreads / 64);
+    const int64_t fixed = sizeof(GroupLds) + sizeof(HitQueue<128>) * (kGroupThreads / 64);
     return V.gmaxw > 1 && ints <= 4096ll * V.gmaxw && fixed + 4 * ints <= kGroupLds;
 }
 

@@ -883,3 +883,42 @@ def test_group_windows_match_oracle_at_the_edges_of_blocks(n, sizes, k, nbins, c
     dlog = []
     E.run_device(40, k=k, log=dlog)
     assert_same_state(E, oe, dlog, olog, (pys, nps))
+
+
+@pytest.mark.parametrize("k", [1, 3, 32])
+def test_batched_replicas_at_the_edges_of_chunks(k):
+    """Replicas around one and two chunks of other atoms, one grid counted in
+    LDS and one past it: every replica equals its independent run."""
+    from fullrmc_amd.Engine import run_replicas
+    boxes = []
+    for i, (n, nbins) in enumerate(((63, 150), (2047, 150), (2048, 150), (2049, 1600), (4096, 150), (4161, 150))):
+        rng = np.random.default_rng(700 + i)
+        L = (n / 0.05) ** (1 / 3)
+        basis = systems.cubic_basis(L) if i % 2 else systems.triclinic_basis(L, 1.1 * L, 1.2 * L, 80, 95, 105)
+        b = dict(real=(rng.random((n, 3)) @ basis.astype(np.float64)).astype(F32),
+                 elements=[("O", "Si")[j] for j in rng.integers(0, 2, n)],
+                 molecules=(np.arange(n) // 3).astype(np.int32), basis=basis, recip=systems.reciprocal(basis))
+        b["exp"] = pdc_target(b, 0.1, 710 + i, 0.025, 7.5 / nbins, nbins)
+        boxes.append(b)
+
+    def engine(b):
+        E = device_engine(b, [PairDistributionConstraint(b["exp"])])
+        E.set_move_generator(TranslationGenerator(0.3))
+        E.set_tolerance(10.0)
+        return E
+
+    reps = [engine(b) for b in boxes]
+    seeds = list(range(720, 720 + len(boxes)))
+    run_replicas(reps, 60, k=k, seeds=seeds)
+    for E, b, seed in zip(reps, boxes, seeds):
+        E.sync_from_device()
+        random.seed(seed)
+        np.random.seed(seed)
+        S = engine(b)
+        S.run_device(60, k=k)
+        S.sync_from_device()
+        assert E.realCoordinates.tobytes() == S.realCoordinates.tobytes()
+        assert np.float32(E.totalStandardError).tobytes() == np.float32(S.totalStandardError).tobytes()
+        assert (E.accepted, E.tolerated) == (S.accepted, S.tolerated)
+        assert E.constraints[0].data["intra"].tobytes() == S.constraints[0].data["intra"].tobytes()
+        assert E.constraints[0].data["inter"].tobytes() == S.constraints[0].data["inter"].tobytes()
