@@ -587,8 +587,8 @@ def full_histogram_record(start, elem, dr, H, with_f64):
     n = len(elem)
     gps, fms, _, sched = gpu_full_histogram(start, elem, dr, H)
     gps0, fms0, _, sched0 = gpu_full_histogram(start, elem, dr, H, autotune=False)
-    # the roofline counts the pairs the kernel evaluated (a cell list skips
-    # pairs in non-neighbouring cells); Gpairs/s stays on N(N-1)/2
+    # the roofline counts the pairs the kernel evaluated (pairs of
+    # distant chunks are skipped); Gpairs/s stays on N(N-1)/2
     ev = sched.get("evaluated_pairs", -1)
     ev = ev if ev > 0 else n * (n - 1) // 2
     tf = ev / (fms * 1e-3) * OPS_PER_PAIR / 1e12
