@@ -193,11 +193,16 @@ __global__ void __launch_bounds__(256) k_ad_chains(const int32_t *__restrict__ i
 // then atoms against the row chunk's box, and queues the pairs within the
 // largest limit; full waves evaluate the queue exactly, in both directions
 // where both atoms are listed.
+// The items grow as the square of the atoms, so the launch is bounded and its
+// waves stride over them: 64 listed atoms of 200,000 take 472 us with at most 16,384
+// workgroups, 497 with 4,096, 513 with 65,536, 1,066 with an item per wave, and from
+// 889,632 atoms on that is more than a launch holds.
+constexpr int64_t kAdBlocks = 1 << 14;
 constexpr int kAdOffsets = 4;  // 13,500 atoms: 155 us a call; 2: 181, 8: 177, 16: 180
 
 template <bool PBC>
-__global__ void __launch_bounds__(256) k_ad_chunks(AdArgs A, AdOut O, ChunkSort S, int32_t nsub,
-                                                   const int32_t *__restrict__ head, const int32_t *__restrict__ next) {
+__global__ void __launch_bounds__(256) k_ad_chunks(AdArgs A, AdOut O, ChunkSort S, const int32_t *__restrict__ head,
+                                                   const int32_t *__restrict__ next) {
     extern __shared__ uint32_t lcnt[];
     __shared__ float4 list_of[4][64];
     __shared__ int32_t pos_of[4][64];
@@ -206,7 +211,7 @@ __global__ void __launch_bounds__(256) k_ad_chunks(AdArgs A, AdOut O, ChunkSort 
     if (O.cnt)
         for (int32_t s = threadIdx.x; s < nws; s += blockDim.x) lcnt[s] = 0;
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     float4 *list = list_of[wave];
     int32_t *pos = pos_of[wave];
     uint32_t *queue = queue_of[wave];
@@ -217,10 +222,10 @@ __global__ void __launch_bounds__(256) k_ad_chunks(AdArgs A, AdOut O, ChunkSort 
     for (int o = 32; o > 0; o >>= 1) range = fmaxf(range, __shfl_xor(range, o));
     const float cut2 = cut_squared(P.C, range, coord_max<PBC>(S.meta));
     const int32_t N = (int32_t)load_dev(S.meta + M_NCHUNK), ndist = N / 2 + 1;
-    const int64_t item = (int64_t)blockIdx.x * 4 + wave;
-    const int32_t sub = (int32_t)(item / N), i = (int32_t)(item % N);
-    const int32_t e0 = sub * kAdOffsets, e1 = min(ndist, e0 + kAdOffsets);
-    if (sub < nsub && e0 < e1) {
+    const int64_t items = (int64_t)N * ((ndist + kAdOffsets - 1) / kAdOffsets);
+    for (int64_t item = (int64_t)blockIdx.x * 4 + wave; item < items; item += (int64_t)gridDim.x * 4) {
+        const int32_t sub = (int32_t)(item / N), i = (int32_t)(item - (int64_t)sub * N);
+        const int32_t e0 = sub * kAdOffsets, e1 = min(ndist, e0 + kAdOffsets);
         const float4 r = S.sx[(int64_t)i * 64 + lane];
         const int bx = __float_as_int(reinterpret_cast<const float *>(S.cbox + kBox * (int64_t)i)[lane & 7]);
         auto of = [&](int k) { return __int_as_float(__builtin_amdgcn_readlane(bx, k)); };
@@ -318,6 +323,7 @@ __global__ void __launch_bounds__(256) k_ad_chunks(AdArgs A, AdOut O, ChunkSort 
             }
         }
         drain(qn);
+        __builtin_amdgcn_wave_barrier();
     }
     if (O.cnt) ad_flush(O, lcnt, nws);
 }
@@ -557,11 +563,11 @@ int ad_run(AdArgs A, float *dintra, float *dinter, int32_t *nintra, int32_t *nin
         k_ad_chains<<<blocks_for(A.k, 256), 256, 0, st>>>(A.indexes, A.k, A.n, head, next);
         FRMC_CHECK_LAUNCH();
     }
-    const int32_t nsub = chunks ? (int32_t)((S.maxchunks / 2 + kAdOffsets) / kAdOffsets) : 0;
+    const int64_t items = chunks ? S.maxchunks * ((S.maxchunks / 2 + kAdOffsets) / kAdOffsets) : 0;
+    const unsigned cblocks = (unsigned)std::min<int64_t>((items + 3) / 4, kAdBlocks);
     auto pass = [&]() {
         if (chunks)
-            k_ad_chunks<SRC == AD_PBC><<<(unsigned)((S.maxchunks * nsub + 3) / 4), 256, lds, st>>>(A, O, S, nsub, head,
-                                                                                                  next);
+            k_ad_chunks<SRC == AD_PBC><<<cblocks, 256, lds, st>>>(A, O, S, head, next);
         else
             k_ad_pass<SRC><<<dim3(nb, (unsigned)((A.k + per - 1) / per)), 256, lds, st>>>(A, O, per);
     };

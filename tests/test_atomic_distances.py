@@ -284,3 +284,32 @@ def test_near_pairs_of_many_atoms_match_oracle(cell, limit):
         ref = refcpu.multiple_atomic_distances_coords(idx, coords, basis, pbc, mol, elem, nel, lo, up, flags,
                                                       allAtoms=allAtoms)
         assert _same(got, ref)
+
+
+def _near(n, idx, box, basis, mol, elem, lo, up, flags):
+    """The oracle's sums for a list, over the atoms that lie within the limits of
+    the list's slab in x alone: the others are in no pair, and the order stays."""
+    dx = np.float64(up.max()) / basis[0, 0] + 1e-5
+    x = box[idx, 0]
+    keep = np.flatnonzero((box[:, 0] >= x.min() - dx) & (box[:, 0] <= x.max() + dx))
+    return refcpu.multiple_atomic_distances_coords(np.searchsorted(keep, idx).astype(np.int32), box[keep], basis, True,
+                                                   mol[keep], elem[keep], 2, lo, up, flags)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(900001, 21), (900001, 9000), (14300001, 1)])
+def test_lists_of_the_largest_boxes_match_oracle(n, k):
+    """Boxes whose pairs of chunks, one to a wave, are more work items than a
+    launch holds, and more workgroups than 32 bits count."""
+    rng = np.random.default_rng(n % 1000 + k)
+    basis = systems.cubic_basis((n / 0.07) ** (1 / 3))
+    box = rng.random((n, 3), F32)
+    box[:, 0] = np.sort(box[:, 0])
+    mol = (np.arange(n) // 3).astype(np.int32)
+    elem = rng.integers(0, 2, n).astype(np.int32)
+    lo, up = _limits(2, 0.0, 2.6, seed=6)
+    idx = rng.permutation(np.arange(n // 2, n // 2 + k)).astype(np.int32)
+    got = gad.multiple_atomic_distances_coords(idx, box, basis, True, mol, elem, 2, lo, up, interMolecular=True,
+                                               intraMolecular=True, countWithinLimits=True)
+    assert got[0].sum() + got[2].sum() > 0
+    assert _same(got, _near(n, idx, box, basis, mol, elem, lo, up, refcpu.ad_flags(True, True, True)))
