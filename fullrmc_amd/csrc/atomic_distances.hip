@@ -508,10 +508,20 @@ struct AdScratch {
     }
 };
 
-// Pairs from which the chunks pay for their sort (five launches and a chain
-// pass, about 25 us): all pairs of 2,048 atoms (3,000 atoms: 138 us against 166;
-// 1,000: 127 without).
+// Whether k listed atoms of n take the chunks.  They pay for their sort (five
+// launches and a chain pass, about 25 us) from all pairs of 2,048 atoms on (3,000
+// atoms: 138 us against 166; 1,000: 127 without).  Their pass tests all pairs of chunks
+// whatever the list: about 55 us + 9e-9 n^2 more than a call's launches, where the
+// direct pass takes k (0.08 + 1.1e-6 n), with limits of 2.6 A, and up to k (0.8 +
+// 1.1e-6 n) at 6 A, where each listed atom has ten times the pairs to sort.  The line
+// is at 0.15: 200,000 atoms, us direct and by chunks at 2.6 A: 84 and 472 for 64
+// listed atoms, 387 and 516 for 1,024, 678 and 524 for 2,048; at 6 A: 136 and 544, 1,191
+// and 759, 2,323 and 1,056; 1,000,000 atoms, 2,048 listed: 2,926 and 8,967.
 constexpr int64_t kChunkPairs = (int64_t)1 << 22;
+
+bool chunks_pay(int64_t k, int64_t n) {
+    return k * n >= kChunkPairs && (double)k * (16e6 + 120.0 * n) >= 6e9 + (double)n * n;
+}
 
 template <int SRC>
 int ad_run(AdArgs A, float *dintra, float *dinter, int32_t *nintra, int32_t *ninter, hipStream_t st) {
@@ -524,7 +534,7 @@ int ad_run(AdArgs A, float *dintra, float *dinter, int32_t *nintra, int32_t *nin
     const int64_t pairs = (int64_t)A.k * A.n;
     // only pairs inside the limits can be skipped by their distance
     const bool chunks = SRC != AD_DISTS && (A.flags & FRMC_AD_WITHIN) && A.indexes && A.nel <= 64 &&
-                        A.n < (1 << 25) && pairs >= kChunkPairs;
+                        A.n < (1 << 25) && chunks_pay(A.k, A.n);
     ChunkSort S;
     memset(&S, 0, sizeof(S));
     if (chunks) S = chunk_layout(A.n);
