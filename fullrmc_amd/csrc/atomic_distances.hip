@@ -659,6 +659,7 @@ extern "C" int frmc_multiple_atomic_distances_coords(const int32_t *indexes, int
                                                      int32_t *nintra, float *dintra, int32_t *ninter, float *dinter,
                                                      void *stream) {
     FRMC_REQUIRE(numberOfElements >= 1 && n >= 0 && nidx >= 0, "atomic_distances: bad sizes");
+    FRMC_REQUIRE(!isPBC || basis, "basis is NULL");
     hipStream_t st = as_stream(stream);
     AdArgs A{};
     A.coords = boxCoords;

@@ -77,3 +77,22 @@ def test_schedule_and_replica_controls_validate_without_gpu():
     steps = ctypes.c_int64(-1)
     _lib.check(L.frmc_replica_batch_times(ms, ctypes.byref(steps)))
     assert steps.value >= 0
+
+
+def test_periodic_calls_without_a_basis_are_refused_on_the_host():
+    """The kernels read the basis from device memory: an address that is not
+    there must not reach them."""
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("libfrmc_hip.so not built")
+    L = _lib.lib()
+    one = ctypes.c_int64(0)
+    a = ctypes.addressof(one)  # never read: the basis is checked first
+    calls = [lambda: L.frmc_multiple_atomic_distances_coords(a, 1, a, 2, None, 1, a, a, 1, a, a, 7, 1, a, a, a, a, None),
+             lambda: L.frmc_multiple_pairs_histograms_coords(a, 1, a, 2, None, 1, a, a, 1, 0.0, 1.0, 0.1, 10, 1, a, a,
+                                                             None),
+             lambda: L.frmc_full_pairs_histograms_coords(a, 2, None, 1, a, a, 1, 0.0, 1.0, 0.1, 10, a, a, None),
+             lambda: L.frmc_full_pairs_counts(a, 2, None, 1, a, a, 1, 0.0, 1.0, 0.1, 10, a, None),
+             lambda: L.frmc_full_pairs_counts_f64(a, 2, None, 1, a, a, 1, 0.0, 1.0, 0.1, 10, a, None, None)]
+    for call in calls:
+        assert call() == 1
+        assert L.frmc_last_error() == b"basis is NULL"
