@@ -445,6 +445,7 @@ __device__ __forceinline__ void full_chunks(const ChunkArgs &K, const Basis &B, 
     int32_t *__restrict__ counts = K.counts;
     extern __shared__ float4 lds4[];
     __shared__ int32_t next;
+    __shared__ unsigned long long all_evaluated;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwave = blockDim.x >> 6;
     char *mine = reinterpret_cast<char *>(lds4) + wave * kWaveLds;
     float4 *lxyz = reinterpret_cast<float4 *>(mine);
@@ -454,7 +455,10 @@ __device__ __forceinline__ void full_chunks(const ChunkArgs &K, const Basis &B, 
     const int32_t size = (int32_t)A.size, H = A.g.H, nel = A.nel;
     const int32_t nbins = LDS_HIST ? (lds_intra ? 2 * size : size) : 0;  // inter-molecular bins first
     for (int32_t s = tid; s < nbins; s += blockDim.x) hist[s] = 0;
-    if (tid == 0) next = 0;
+    if (tid == 0) {
+        next = 0;
+        all_evaluated = 0;
+    }
     __syncthreads();
 
     const int32_t N = (int32_t)load_dev(meta + M_NCHUNK);
@@ -684,8 +688,11 @@ __device__ __forceinline__ void full_chunks(const ChunkArgs &K, const Basis &B, 
     if (lost) atomicAdd(&counts[2 * A.size], lost);
     if (EDGE && nre)
         atomicAdd(reinterpret_cast<unsigned long long *>(&counts[2 * A.size + 2]), (unsigned long long)nre);
-    if (K.count_pairs && lane == 0)
-        atomicAdd(reinterpret_cast<unsigned long long *>(&meta[M_PAIRS]), evaluated * 64ull);
+    if (K.count_pairs) {  // one atomic per workgroup (one per wave: about 60 us more at 13,500 atoms)
+        if (lane == 0) atomicAdd(&all_evaluated, evaluated * 64ull);
+        __syncthreads();
+        if (tid == 0) atomicAdd(reinterpret_cast<unsigned long long *>(&meta[M_PAIRS]), all_evaluated);
+    }
     if (LDS_HIST) {
         __syncthreads();
         int32_t *dst = K.partial + (int64_t)blockIdx.x * nbins;
@@ -741,6 +748,11 @@ __global__ void __launch_bounds__(1024) k_chunk_finish(const int32_t *__restrict
         }
     }
     if (overflow && blockIdx.x == 0 && threadIdx.x == 0) *overflow = load_dev(counts + 2 * size);
+}
+
+// the number of evaluated pairs to a host word
+__global__ void k_chunk_pairs(const uint32_t *__restrict__ meta, int64_t *pairs) {
+    if (threadIdx.x == 0) *pairs = load_dev(reinterpret_cast<const int64_t *>(meta + M_PAIRS));
 }
 
 // Bounds of the approximate bin t = (v_sqrt(s) - min) * (1/bin) against the
@@ -905,7 +917,7 @@ int run_chunks(const ChunkRun &R, const float *coords, int32_t n, const float *d
     K.A = A;
     K.F = fast_bin(A, E, isPBC);
     K.lds_intra = nbins == 2 * size;
-    K.count_pairs = timing_enabled() && R.pairs;
+    K.count_pairs = R.pairs != nullptr;
     K.partial = (int32_t *)(scr + o_part);
     K.counts = counts;
 #define FRMC_CHUNKS(P, L, ED)                                                                                     \
@@ -933,11 +945,8 @@ int run_chunks(const ChunkRun &R, const float *coords, int32_t n, const float *d
         k_chunk_finish<<<(unsigned)((2 * size + 63) / 64), 1024, 0, st>>>(
             K.partial, (int32_t)blocks, nbins, size, counts, R.counts ? nullptr : R.hintra,
             R.counts ? nullptr : R.hinter, R.overflow);
+    if (R.pairs) k_chunk_pairs<<<1, 64, 0, st>>>(S.meta, R.pairs);
     e = hipGetLastError();
-    if (e == hipSuccess && K.count_pairs) {
-        e = hipMemcpyAsync(R.pairs, S.meta + M_PAIRS, sizeof(int64_t), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-    }
     (void)hipFreeAsync(scr, st);
     if (e != hipSuccess) {
         set_error("full histogram launch failed: %s", hipGetErrorString(e));

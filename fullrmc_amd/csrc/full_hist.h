@@ -76,7 +76,7 @@ struct ChunkRun {
     int32_t *used_nt = nullptr; // threads launched
     int32_t per_cu = 0;         // workgroups per CU, 0: as many as fit
     int64_t *blocks = nullptr;  // workgroups launched
-    int64_t *pairs = nullptr;   // pairs evaluated, filled only while timing is on
+    int64_t *pairs = nullptr;   // host word for the pairs evaluated, or null: not counted
     // the result: added into counts ([2][nel][nel][H], overflow, re-checks),
     // or written as the float32 histograms, the lost pairs to a host word
     int32_t *counts = nullptr;

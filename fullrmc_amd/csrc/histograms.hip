@@ -458,7 +458,6 @@ static thread_local FullChoice g_last;     // frmc_last_full_schedule (per threa
 static thread_local int64_t g_last_blocks = 0;
 static thread_local int g_last_tuned = 0;
 static thread_local int64_t g_last_evaluated = -1;  // pairs evaluated by the last call (-1: not measured)
-static thread_local int64_t g_chunks_evaluated = -1;  // set by run_chunks when timing is on
 static std::mutex g_tune_mu;
 // shape class -> tuned schedule.  Class: device, floor(log2 n), bins
 // (2*nel*nel*H), boundary kind (0 none, 1 triclinic, 2 orthorhombic), EDGE.
@@ -471,7 +470,7 @@ static double range_of(const HistArgs &A, const Edge64 *E) {
 
 static int run_full(const FullChoice &C, const float *coords, int32_t n, const Basis &B, int isPBC, bool ortho,
                     const int32_t *mol, const int32_t *elem, const HistArgs &A, const Edge64 *E, int ncu,
-                    int32_t *counts, hipStream_t st, int64_t *nblocks) {
+                    int32_t *counts, hipStream_t st, int64_t *nblocks, int64_t *pairs) {
     if (C.cells) {
         int32_t m[3];
         if (!isPBC || !cell_grid(B, range_of(A, E), m)) {
@@ -484,9 +483,8 @@ static int run_full(const FullChoice &C, const float *coords, int32_t n, const B
         R.nt = C.nt;
         R.per_cu = C.per_cu;
         R.blocks = nblocks;
-        R.pairs = &g_chunks_evaluated;
+        R.pairs = pairs;
         R.counts = counts;
-        g_chunks_evaluated = -1;
         return run_chunks(R, coords, n, nullptr, B, isPBC, mol, elem, A, E, ncu, st);
     }
     const size_t lds_bytes = sizeof(int32_t) * 2 * A.size;
@@ -578,7 +576,7 @@ static int tune_full(const float *coords, int32_t n, const Basis &B, int isPBC, 
             k_fill_i32<<<64, 256, 0, st>>>(scratch, len, 0);
             if (hipEventRecord(ev[4 * c + 2 * rep], st) != hipSuccess) rc = FRMC_EHIP;
             if (rc == FRMC_OK)
-                rc = run_full(cand[c], coords, n, B, isPBC, ortho, mol, elem, A, E, ncu, scratch, st, nullptr);
+                rc = run_full(cand[c], coords, n, B, isPBC, ortho, mol, elem, A, E, ncu, scratch, st, nullptr, nullptr);
             if (rc == FRMC_OK && hipEventRecord(ev[4 * c + 2 * rep + 1], st) != hipSuccess) rc = FRMC_EHIP;
             if (rc == FRMC_EHIP) set_error("hipEventRecord failed while tuning");
         }
@@ -649,25 +647,37 @@ static bool chunk_route(int32_t n, const HistArgs &A) {
     return !g_forced_on && g_autotune && chunks_take(n, A);
 }
 
-// HIP events around the pass when per-thread timing is on (frmc_set_timing)
+// HIP events around the pass when per-thread timing is on (frmc_set_timing); the
+// pass then gets a host word for the number of pairs it evaluates, which its last
+// kernel writes (a copy that waits would be timed with it: 0.200 ms for a
+// histogram whose whole call takes 0.097).  evaluated: that number, else -1.
 template <typename Pass>
-static int timed_pass(hipStream_t st, Pass pass) {
-    if (!timing_enabled()) return pass();
+static int timed_pass(hipStream_t st, int64_t &evaluated, Pass pass) {
+    evaluated = -1;
+    if (!timing_enabled()) return pass(nullptr);
+    HostWords pairs(st);
+    if (!pairs.p) {
+        set_error("allocation of pinned host words failed");
+        return FRMC_ENOMEM;
+    }
+    pairs.p[0] = -1;
     hipEvent_t a = nullptr, b = nullptr;
     FRMC_CHECK_HIP(hipEventCreate(&a));
     FRMC_CHECK_HIP(hipEventCreate(&b));
     FRMC_CHECK_HIP(hipEventRecord(a, st));
-    int rc = pass();
+    int rc = pass(pairs.p);
     float ms = 0.f;
     hipError_t e = hipEventRecord(b, st);
     if (e == hipSuccess) e = hipEventSynchronize(b);
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, a, b);
+    if (e == hipSuccess) e = pairs.wait();
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
     if (e != hipSuccess && rc == FRMC_OK) {
         set_error("kernel timing failed: %s", hipGetErrorString(e));
         rc = FRMC_EHIP;
     }
+    if (e == hipSuccess) evaluated = pairs.p[0];
     set_last_kernel_ms(ms);
     return rc;
 }
@@ -689,15 +699,17 @@ static int full_by_chunks(ChunkRun R, const float *coords, int32_t n, const floa
     int32_t nt = 0;
     R.blocks = &blocks;
     R.used_nt = &nt;
-    R.pairs = &g_chunks_evaluated;
-    g_chunks_evaluated = -1;
-    const int rc = timed_pass(st, [&] { return run_chunks(R, coords, n, dbasis, hB, isPBC, mol, elem, A, E, ncu, st); });
+    int64_t evaluated = -1;
+    const int rc = timed_pass(st, evaluated, [&](int64_t *pairs) {
+        R.pairs = pairs;
+        return run_chunks(R, coords, n, dbasis, hB, isPBC, mol, elem, A, E, ncu, st);
+    });
     g_last = FullChoice();
     g_last.nt = nt;
     g_last.R = 1;  // one row atom per thread
     g_last_blocks = blocks;
     g_last_tuned = 1;
-    g_last_evaluated = g_chunks_evaluated;
+    g_last_evaluated = evaluated;
     return rc;
 }
 
@@ -720,13 +732,14 @@ static int launch_full_timed(const float *coords, int32_t n, const Basis &B, int
     FullChoice C;
     int tuned = 0;
     if (int rc = choose_full(coords, n, B, isPBC, ortho, mol, elem, A, E, dev, ncu, st, C, tuned)) return rc;
-    int64_t blocks = 0;
-    const int rc = timed_pass(
-        st, [&] { return run_full(C, coords, n, B, isPBC, ortho, mol, elem, A, E, ncu, counts, st, &blocks); });
+    int64_t blocks = 0, evaluated = -1;
+    const int rc = timed_pass(st, evaluated, [&](int64_t *pairs) {
+        return run_full(C, coords, n, B, isPBC, ortho, mol, elem, A, E, ncu, counts, st, &blocks, pairs);
+    });
     g_last = C;
     g_last_blocks = blocks;
     g_last_tuned = tuned;
-    g_last_evaluated = C.cells ? g_chunks_evaluated : (int64_t)n * (n - 1) / 2;
+    g_last_evaluated = C.cells && chunks_take(n, A) ? evaluated : (int64_t)n * (n - 1) / 2;
     return rc;
 }
 

@@ -3,10 +3,13 @@ all-pairs loops: partly filled chunks and columns, odd and even chunk
 numbers, cubic, triclinic and flat cells, open boundaries, coordinates in other
 images, bins in LDS, in global memory and past the end of the array, and the
 binary64 recompute with its count of re-checked pairs."""
+import ctypes
+import time
+
 import numpy as np
 import pytest
 
-from fullrmc_amd import systems, tuning
+from fullrmc_amd import _lib, systems, tuning
 from fullrmc_amd.Core import pairs_histograms as gph
 from oracle import refcpu
 
@@ -97,3 +100,37 @@ def test_coordinates_that_are_not_finite_are_never_in_range():
     keep = np.all(np.isfinite(coords), axis=1)
     want = refcpu.full_pairs_histograms_coords(coords[keep], basis, True, mol[keep], elem[keep], *grid, ncores=8)
     assert got[0].tobytes() == want[0].tobytes() and got[1].tobytes() == want[1].tobytes()
+
+
+def test_kernel_time_holds_no_wait_for_the_host():
+    """frmc_last_kernel_ms covers the pass alone, so it is not above the whole call's
+    time without timing; the evaluated pairs are counted all the same."""
+    import torch
+    rng = np.random.default_rng(6)
+    n, H, L = 13500, 1000, _lib.lib()
+    dev = [torch.from_numpy(a).cuda() for a in
+           (rng.random((n, 3), F32), np.diag([45.0, 45.0, 90.0]).astype(F32), np.arange(n, dtype=np.int32) // 3,
+            rng.integers(0, 2, n).astype(np.int32), np.zeros((2, 2, 2, H), F32))]
+    c, b, m, e, out = (t.data_ptr() for t in dev)
+
+    def call():
+        t0 = time.perf_counter()
+        _lib.check(L.frmc_full_pairs_histograms_coords(c, n, b, 1, m, e, 2, 0.0, 20.0, 0.02, H, out, out + 16 * H,
+                                                       torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return time.perf_counter() - t0
+
+    whole = min(call() for _ in range(20))
+    evaluated = ctypes.c_int64(0)
+    L.frmc_set_timing(1)
+    try:
+        kernel = []
+        for _ in range(20):
+            call()
+            kernel.append(L.frmc_last_kernel_ms() * 1e-3)
+        _lib.check(L.frmc_last_full_evaluated(ctypes.byref(evaluated)))
+    finally:
+        L.frmc_set_timing(0)
+    counted = int(dev[4].sum().item())
+    assert counted <= evaluated.value <= n * n
+    assert min(kernel) < 1.3 * whole, (min(kernel), whole)
