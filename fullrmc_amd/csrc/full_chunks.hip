@@ -271,6 +271,10 @@ __global__ void __launch_bounds__(256) k_chunk_scatter(const float *__restrict__
 // call's time: 1,000 atoms in 52 us against 62, 4,000 in 64 against 67; at 13,500
 // the one workgroup would take longer than the launches it saves.
 constexpr int32_t kSmallSort = 4096;
+// Words of counts that the one workgroup clears besides; beyond, the launches that
+// clear with the whole chip: 1,000 atoms of 64 elements, 1,000 bins (8.2 million words)
+// 114 us a call against 540, of 20 elements, 2,000 bins 97 against 167.
+constexpr int64_t kSmallClear = 1 << 16;
 
 template <bool PBC>
 __global__ void __launch_bounds__(1024) k_chunk_sort_small(const float *__restrict__ dbasis, Basis hB,
@@ -750,6 +754,20 @@ __global__ void __launch_bounds__(1024) k_chunk_finish(const int32_t *__restrict
     if (overflow && blockIdx.x == 0 && threadIdx.x == 0) *overflow = load_dev(counts + 2 * size);
 }
 
+// k_chunk_finish without partials: counts made by atomics, as float32.  Bound by
+// its reads and writes (16 waves per 64 slots, as for partials, took about 150 us
+// more at 8.2 million slots).
+__global__ void __launch_bounds__(256) k_chunk_convert(const int32_t *__restrict__ counts, int64_t size,
+                                                       float *__restrict__ hintra, float *__restrict__ hinter,
+                                                       int64_t *overflow) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *overflow = load_dev(counts + 2 * size);
+    for (int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x; s < 2 * size; s += (int64_t)gridDim.x * 256) {
+        const float f = (float)counts[s];
+        if (s < size) hintra[s] = f;
+        else hinter[s - size] = f;
+    }
+}
+
 // the number of evaluated pairs to a host word
 __global__ void k_chunk_pairs(const uint32_t *__restrict__ meta, int64_t *pairs) {
     if (threadIdx.x == 0) *pairs = load_dev(reinterpret_cast<const int64_t *>(meta + M_PAIRS));
@@ -819,10 +837,11 @@ void launch_chunk_sort(ChunkSort &S, char *scr, const float *coords, int32_t n, 
             *base = (int32_t *)(scr + S.o_base);
     int2 *where = (int2 *)(scr + S.o_where);
     const unsigned nb = blocks_for(n, 256), cb = (unsigned)((S.maxchunks + 3) / 4);
-    if (n <= kSmallSort && isPBC) {
+    const bool small = n <= kSmallSort && nzero <= kSmallClear;
+    if (small && isPBC) {
         k_chunk_sort_small<true><<<1, 1024, 0, st>>>(dbasis, hB, coords, n, mol, elem, nel, meta, where, sx, smol, zero,
                                                      nzero);
-    } else if (n <= kSmallSort) {
+    } else if (small) {
         k_chunk_sort_small<false><<<1, 1024, 0, st>>>(dbasis, hB, coords, n, mol, elem, nel, meta, where, sx, smol, zero,
                                                       nzero);
     } else {
@@ -941,7 +960,10 @@ int run_chunks(const ChunkRun &R, const float *coords, int32_t n, const float *d
     }
 #undef FRMC_CHUNKS_ED
 #undef FRMC_CHUNKS
-    if (nbins || !R.counts)
+    if (!nbins && !R.counts)
+        k_chunk_convert<<<std::min(2048u, blocks_for(2 * size, 256)), 256, 0, st>>>(counts, size, R.hintra, R.hinter,
+                                                                                    R.overflow);
+    else if (nbins)
         k_chunk_finish<<<(unsigned)((2 * size + 63) / 64), 1024, 0, st>>>(
             K.partial, (int32_t)blocks, nbins, size, counts, R.counts ? nullptr : R.hintra,
             R.counts ? nullptr : R.hinter, R.overflow);

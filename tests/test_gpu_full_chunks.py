@@ -134,3 +134,32 @@ def test_kernel_time_holds_no_wait_for_the_host():
     counted = int(dev[4].sum().item())
     assert counted <= evaluated.value <= n * n
     assert min(kernel) < 1.3 * whole, (min(kernel), whole)
+
+
+@pytest.mark.parametrize("n", [100, 1000, 4096])
+def test_few_atoms_of_many_elements(n):
+    """Up to 64 elements of 1,000 bins: the counts are cleared and converted by the
+    whole chip (in the one workgroup that sorts few atoms: ten times the time of 2
+    elements at 1,000 atoms, now 2.3 times)."""
+    import torch
+    coords, basis, mol, rng = box(n, "triclinic", 8, True)
+    grid = (F32(0.0), F32(9.0), F32(0.009), 1000)
+    best = {}
+    for nel in (2, 6, 64):
+        elem = rng.integers(0, nel, n).astype(np.int32)
+        ri, re_ = refcpu.full_pairs_histograms_coords(coords, basis, True, mol, elem, nel, *grid, ncores=8)
+        gi, ge = gph.full_pairs_histograms_coords(coords, basis, True, mol, elem, nel, *grid)
+        assert gi.tobytes() == ri.tobytes() and ge.tobytes() == re_.tobytes()
+        dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (coords, basis, mol, elem)]
+        out = torch.empty((2, nel, nel, 1000), device="cuda")
+        c, b, m, e = (t.data_ptr() for t in dev)
+        times = []
+        for _ in range(12):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            _lib.check(_lib.lib().frmc_full_pairs_histograms_coords(
+                c, n, b, 1, m, e, nel, *grid, out[0].data_ptr(), out[1].data_ptr(),
+                torch.cuda.current_stream().cuda_stream))
+            times.append(time.perf_counter() - t0)
+        best[nel] = min(times)
+    assert best[64] < 5 * best[2], best
