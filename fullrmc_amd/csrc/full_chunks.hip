@@ -285,7 +285,8 @@ __global__ void __launch_bounds__(1024) k_chunk_sort_small(const float *__restri
                                                            float4 *__restrict__ sx, int32_t *__restrict__ smol,
                                                            int32_t *__restrict__ counts, int64_t ncounts) {
     constexpr int kCols = kSmallSort / 96 + 1;
-    __shared__ int32_t cell[kCols * kNZ], tot[kCols], base[kCols];
+    __shared__ __align__(8) int32_t cell[kCols * kNZ];  // read as pairs below
+    __shared__ int32_t tot[kCols], base[kCols];
     __shared__ uint32_t amax, ext[6];
     __shared__ ChunkPlan P;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -875,7 +876,7 @@ int run_chunks(const ChunkRun &R, const float *coords, int32_t n, const float *d
     ChunkSort S = chunk_layout(n);
     const int64_t maxchunks = S.maxchunks;
     // bins in LDS: both halves, else the inter-molecular half, else none
-    const size_t kMaxHist = 112 * 1024;  // leaves eight waves' lists of the 160 KB
+    const size_t kMaxHist = 112 * 1024;  // leaves sixteen waves' lists (42 KB) of the 160 KB
     const int64_t size = A.size;
     const int64_t nbins = sizeof(int32_t) * 2 * size <= kMaxHist ? 2 * size
                           : sizeof(int32_t) * size <= kMaxHist   ? size
