@@ -369,14 +369,21 @@ void launch_sq_exact(const float *G, int32_t k, int32_t H, const float *M, int32
 
 // Waves per workgroup: eight while the tiles do not fill the chip by themselves
 // (2,000 r, 1,000 Q: 64 curves 12.0 us against 13.5 with four and with sixteen),
-// four beyond (256 curves: 22.4 us against 24.3).
+// four beyond (256 curves: 22.4 us against 24.3).  A launch takes the curves of as
+// many tiles as a grid has rows; more curves take more launches.
+constexpr int32_t kTileRows = 65535;
+constexpr int64_t kMaxCurves = 64 * 65535;  // of a call
+
 void launch_sq_mfma(const float *G, int32_t k, int32_t H, const float *M, int32_t nQ, int32_t addOne, float *S,
                     hipStream_t st) {
-    const dim3 grid((unsigned)((nQ + kTQ - 1) / kTQ), (unsigned)((k + kTP - 1) / kTP));
-    if ((int64_t)grid.x * grid.y > 256)
-        k_sq_mfma<4><<<grid, 256, 0, st>>>(G, k, H, M, nQ, addOne, S);
-    else
-        k_sq_mfma<8><<<grid, 512, 0, st>>>(G, k, H, M, nQ, addOne, S);
+    for (int64_t p = 0; p < k; p += (int64_t)kTileRows * kTP) {
+        const int32_t kp = (int32_t)std::min<int64_t>(k - p, (int64_t)kTileRows * kTP);
+        const dim3 grid((unsigned)((nQ + kTQ - 1) / kTQ), (unsigned)((kp + kTP - 1) / kTP));
+        if ((int64_t)grid.x * grid.y > 256)
+            k_sq_mfma<4><<<grid, 256, 0, st>>>(G + p * H, kp, H, M, nQ, addOne, S + p * nQ);
+        else
+            k_sq_mfma<8><<<grid, 512, 0, st>>>(G + p * H, kp, H, M, nQ, addOne, S + p * nQ);
+    }
 }
 
 // reciprocal_space.pyx:89-122: sq = ones; sq[q] += dr*(sin(q*r)/q)*Gr[r]
@@ -521,7 +528,7 @@ extern "C" int frmc_sq_transform(const float *Gr, int32_t k, int32_t H, const fl
     if (mode == FRMC_SQ_EXACT)
         FRMC_REQUIRE(k <= 65535, "sq_transform: at most 65535 curves per call");
     else
-        FRMC_REQUIRE((k + 63) / 64 <= 65535, "sq_transform: too many curves per call");
+        FRMC_REQUIRE(k <= kMaxCurves, "sq_transform: too many curves per call");
     FRMC_CHECK_HIP(timer.start(st));
     if (mode == FRMC_SQ_EXACT) launch_sq_exact(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
     else launch_sq_mfma(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
@@ -532,10 +539,11 @@ extern "C" int frmc_sq_transform(const float *Gr, int32_t k, int32_t H, const fl
 
 // ------------------------------------------------- no-allocation variant
 //
-// Neither mode of the transform allocates.  The entry keeps the limit it has
-// had: matrix-core shapes whose r range, split over about 1,024 tiles of
-// 64 x 64, would give more than 2^22 partial floats are refused.
-constexpr int64_t kSqScratchFloats = (int64_t)1 << 22;
+// Neither mode of the transform allocates.  The entry keeps the limit on
+// matrix-core shapes that it has had: the curves' and Q points' tiles of 64 x 64,
+// times as many parts of the r range (of 64 rows or more) as make about 1,024 of
+// them, hold at most 2^22 results.
+constexpr int64_t kNoallocResults = (int64_t)1 << 22;
 
 extern "C" int frmc_sq_transform_noalloc(const float *Gr, int32_t k, int32_t H, const float *sqMatrix, int32_t nQ,
                                          int addOne, int mode, float *Sq, void *stream) {
@@ -552,15 +560,14 @@ extern "C" int frmc_sq_transform_noalloc(const float *Gr, int32_t k, int32_t H, 
         return FRMC_OK;
     }
     const int64_t bq = (nQ + 63) / 64, bp = (k + 63) / 64, chunks = (H + 63) / 64;
-    FRMC_REQUIRE(bp <= 65535, "sq_transform_noalloc: too many curves per call");
-    int64_t nsplit = std::max<int64_t>(1, std::min<int64_t>((1024 + bq * bp - 1) / (bq * bp), chunks));
-    const int64_t per = ((chunks + nsplit - 1) / nsplit) * 64;
-    nsplit = (H + per - 1) / per;
-    const int64_t need = nsplit * (int64_t)k * nQ;
-    FRMC_REQUIRE(nsplit == 1 || need <= kSqScratchFloats,
-                 "sq_transform_noalloc: k=%d, H=%d, nQ=%d need %lld floats of split partials; the "
-                 "no-allocation entry takes at most %lld: use frmc_sq_transform",
-                 k, H, nQ, (long long)need, (long long)kSqScratchFloats);
+    FRMC_REQUIRE(k <= kMaxCurves, "sq_transform_noalloc: too many curves per call");
+    int64_t parts = std::max<int64_t>(1, std::min<int64_t>((1024 + bq * bp - 1) / (bq * bp), chunks));
+    const int64_t per = ((chunks + parts - 1) / parts) * 64;
+    parts = (H + per - 1) / per;
+    FRMC_REQUIRE(parts == 1 || parts * k * nQ <= kNoallocResults,
+                 "sq_transform_noalloc: k=%d, H=%d, nQ=%d is past this entry's limit of matrix-core shapes "
+                 "(%lld parts of the r range, %lld results in all, at most %lld): use frmc_sq_transform",
+                 k, H, nQ, (long long)parts, (long long)(parts * k * nQ), (long long)kNoallocResults);
     launch_sq_mfma(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
     FRMC_CHECK_LAUNCH();
     return FRMC_OK;

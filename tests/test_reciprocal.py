@@ -182,3 +182,23 @@ def test_sq_transform_edges_of_tiles(k, H, nQ):
     exact, terms = G.astype(np.float64) @ M.astype(np.float64), np.abs(G).astype(np.float64) @ np.abs(M)
     # at most H roundings of 2^-24 relative to the sum of magnitudes, plus the products'
     assert np.all(np.abs(T - exact) <= (H + 1) * 2.0 ** -24 * terms)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [2097120, 2097153, 4194240])
+def test_mfma_curves_past_the_rows_of_a_grid(k):
+    """More curves than the tiles of one launch hold, up to the most that a call
+    takes: each curve within float32 rounding, the ones after the first launch too;
+    one more is refused."""
+    from fullrmc_amd import _device as D, _lib
+    rng = np.random.default_rng(k % 97)
+    H, nQ = 5, 3
+    G = rng.standard_normal((k, H)).astype(F32)
+    M = rng.standard_normal((H, nQ)).astype(F32)
+    S = grs.sq_transform(G, M, addOne=True, mode="mfma").astype(np.float64)
+    exact, terms = G.astype(np.float64) @ M.astype(np.float64) + 1.0, np.abs(G).astype(np.float64) @ np.abs(M) + 1.0
+    assert np.all(np.abs(S - exact) <= (H + 2) * 2.0 ** -24 * terms)
+    if k == 4194240:
+        d = D.empty((1,), F32)  # refused before anything is read
+        for f in (_lib.lib().frmc_sq_transform, _lib.lib().frmc_sq_transform_noalloc):
+            assert f(d.data_ptr(), k + 1, H, d.data_ptr(), nQ, 1, 1, d.data_ptr(), D.stream()) == 1
