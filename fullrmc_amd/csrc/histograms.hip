@@ -456,7 +456,7 @@ static FullChoice g_forced;                // frmc_force_full_schedule (R == 0: 
 static bool g_forced_on = false;
 static thread_local FullChoice g_last;     // frmc_last_full_schedule (per thread)
 static thread_local int64_t g_last_blocks = 0;
-static thread_local int g_last_tuned = 0;
+static thread_local int g_last_tuned = 0;  // 1 by the tuner, 2 the chunk pass by its rule
 static thread_local int64_t g_last_evaluated = -1;  // pairs evaluated by the last call (-1: not measured)
 static std::mutex g_tune_mu;
 // shape class -> tuned schedule.  Class: device, floor(log2 n), bins
@@ -708,7 +708,7 @@ static int full_by_chunks(ChunkRun R, const float *coords, int32_t n, const floa
     g_last.nt = nt;
     g_last.R = 1;  // one row atom per thread
     g_last_blocks = blocks;
-    g_last_tuned = 1;
+    g_last_tuned = 2;
     g_last_evaluated = evaluated;
     return rc;
 }
@@ -737,9 +737,10 @@ static int launch_full_timed(const float *coords, int32_t n, const Basis &B, int
         return run_full(C, coords, n, B, isPBC, ortho, mol, elem, A, E, ncu, counts, st, &blocks, pairs);
     });
     g_last = C;
+    g_last.cells = C.cells && chunks_take(n, A);
     g_last_blocks = blocks;
     g_last_tuned = tuned;
-    g_last_evaluated = C.cells && chunks_take(n, A) ? evaluated : (int64_t)n * (n - 1) / 2;
+    g_last_evaluated = g_last.cells ? evaluated : (int64_t)n * (n - 1) / 2;
     return rc;
 }
 

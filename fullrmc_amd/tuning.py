@@ -40,11 +40,12 @@ def force_full_schedule(threads=None, rowAtoms=None, workgroupsPerCU=None):
 
 
 def last_full_schedule():
-    """The schedule of this thread's last full-histogram call (the chunk-pruned
-    kernel by rule: one row atom per thread, ``tuned``)."""
+    """The schedule of this thread's last full-histogram call.  ``chunks``: the
+    chunk-pruned kernel, ``cells`` if forced, else by its rule (one row atom per
+    thread; ``tuned``, as tuning is on, though nothing was timed)."""
     t, r, tuned = ctypes.c_int32(0), ctypes.c_int32(0), ctypes.c_int32(0)
     w = ctypes.c_int64(0)
     _lib.check(_lib.lib().frmc_last_full_schedule(ctypes.byref(t), ctypes.byref(r), ctypes.byref(w),
                                                   ctypes.byref(tuned)))
     return {"threads": t.value, "rowAtoms": r.value, "workgroups": w.value, "tuned": bool(tuned.value),
-            "cells": r.value == -1}
+            "cells": r.value == -1, "chunks": tuned.value == 2 or r.value == -1}

@@ -66,7 +66,8 @@ float frmc_last_kernel_ms(void);
    tuned classes.  frmc_force_full_schedule pins one schedule for every call
    (rowAtoms == 0 releases it).  frmc_last_full_schedule reports the
    schedule of this thread's last full-histogram call (tuned = 1 when it came
-   from the tuner or the chunk-pruned kernel's rule, whose row atoms are 1). */
+   from the tuner, 2 for the chunk-pruned kernel by its rule, whose row atoms are
+   1, else 0). */
 void frmc_set_autotune(int enable);
 int frmc_force_full_schedule(int32_t threads, int32_t rowAtoms, int32_t workgroupsPerCU);
 int frmc_last_full_schedule(int32_t *threads, int32_t *rowAtoms, int64_t *workgroups, int32_t *tuned);

@@ -166,3 +166,40 @@ def test_cell_list_schedule_refused_on_a_small_cell(si_o):
     with pytest.raises(Exception):
         gph.full_pairs_histograms_coords(si_o["box"], si_o["basis"], True, si_o["mol"], si_o["elem"], 2, F32(0.0),
                                          F32(20.0), F32(0.02), 1000)
+
+
+@pytest.mark.parametrize("H", [2, 30])  # bins in LDS and in global memory
+@pytest.mark.parametrize("boundary", ["orthorhombic", "triclinic", "open"])
+def test_tuner_times_the_all_pairs_kernels_past_64_elements(H, boundary):
+    """65 elements do not fit the chunk pass: by default the first call of a class
+    times the all-pairs schedules, the next reuses the fastest, and with tuning off the
+    rule is taken; 64 elements take the chunk pass.  All equal the oracle."""
+    n = 5003
+    rng = np.random.default_rng(H)
+    basis = systems.cubic_basis(42.0) if boundary == "orthorhombic" else systems.triclinic_basis(40.0, 43.0, 46.0, 75.0,
+                                                                                                95.0, 110.0)
+    coords = (rng.random((n, 3)) * (42.0 if boundary == "open" else 1.0)).astype(F32)
+    mol = (np.arange(n) // 4).astype(np.int32)
+    elem = rng.integers(0, 64, n).astype(np.int32)
+    elem[7] = 64
+    args = (coords, basis, boundary != "open", mol, elem, 65, F32(0.0), F32(9.0), F32(9.0 / H), H)
+    want = refcpu.full_pairs_histograms_coords(*args, ncores=8)
+    tuning.set_autotune(True, forget=True)
+    seen = []
+    for _ in range(2):
+        got = gph.full_pairs_histograms_coords(*args)
+        assert same(got[0], want[0]) and same(got[1], want[1])
+        seen.append(tuning.last_full_schedule())
+    assert seen[0] == seen[1] and seen[0]["tuned"] and not seen[0]["chunks"]
+    tuning.set_autotune(False)
+    got = gph.full_pairs_histograms_coords(*args)
+    assert same(got[0], want[0]) and same(got[1], want[1])
+    fixed = tuning.last_full_schedule()
+    assert not fixed["tuned"] and not fixed["chunks"]
+    tuning.set_autotune(True)
+    elem[7] = 63
+    args = args[:5] + (64,) + args[6:]
+    want = refcpu.full_pairs_histograms_coords(*args, ncores=8)
+    got = gph.full_pairs_histograms_coords(*args)
+    assert same(got[0], want[0]) and same(got[1], want[1])
+    assert tuning.last_full_schedule()["chunks"]
