@@ -356,3 +356,33 @@ def test_short_lists_of_large_boxes_cost_what_the_list_costs():
         return min(times)
 
     assert best(64) < 4 * best(13)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pbc", [True, False])
+@pytest.mark.parametrize("case", ["coordinates", "upper nan", "upper inf", "upper negative", "lower nan"])
+def test_values_that_are_not_finite_by_chunks_and_directly(case, pbc):
+    """2,100 atoms, all of them listed (the chunks, which then cut nothing) and 13
+    (directly): coordinates and limits that are not numbers, infinite or below zero
+    select what the oracle's comparisons select."""
+    rng = np.random.default_rng(11)
+    n, nel = 2100, 3
+    basis = systems.cubic_basis(31.0)
+    box = (rng.random((n, 3)) * (1.0 if pbc else 31.0)).astype(F32)
+    lo, up = _limits(nel, 0.0, 2.6, seed=7)
+    if case == "coordinates":
+        box[17], box[400, 1], box[1999, 2], box[700, 0] = np.nan, np.inf, -np.inf, 3e38
+    else:
+        a = up if case.startswith("upper") else lo
+        a[0, 1] = {"nan": np.nan, "inf": np.inf, "negative": -2.0}[case.split()[1]]
+    mol = rng.integers(0, 500, n).astype(np.int32)
+    elem = rng.integers(0, nel, n).astype(np.int32)
+    few = np.array([17, 3, 400, 1999, 700, 5, 5, 1001, 2099, 0, 64, 63, 1200], np.int32)
+    for idx, allAtoms in ((np.arange(n, dtype=np.int32), True), (few, True), (few, False)):
+        got = gad.multiple_atomic_distances_coords(idx, box, basis, pbc, mol, elem, nel, lo, up, allAtoms=allAtoms)
+        ref = refcpu.multiple_atomic_distances_coords(idx, box, basis, pbc, mol, elem, nel, lo, up, refcpu.ad_flags(),
+                                                      allAtoms=allAtoms)
+        assert got[0].sum() + got[2].sum() > 0
+        for g, r in zip(got, ref):
+            assert np.array_equal(np.isnan(g), np.isnan(r))
+            assert np.where(np.isnan(g), 0, g).tobytes() == np.where(np.isnan(r), 0, r).tobytes()
