@@ -222,9 +222,12 @@ __global__ void __launch_bounds__(256) k_ad_chunks(AdArgs A, AdOut O, ChunkSort 
     for (int o = 32; o > 0; o >>= 1) range = fmaxf(range, __shfl_xor(range, o));
     const float cut2 = cut_squared(P.C, range, coord_max<PBC>(S.meta));
     const int32_t N = (int32_t)load_dev(S.meta + M_NCHUNK), ndist = N / 2 + 1;
-    const int64_t items = (int64_t)N * ((ndist + kAdOffsets - 1) / kAdOffsets);
-    for (int64_t item = (int64_t)blockIdx.x * 4 + wave; item < items; item += (int64_t)gridDim.x * 4) {
-        const int32_t sub = (int32_t)(item / N), i = (int32_t)(item - (int64_t)sub * N);
+    const int32_t nsub = (ndist + kAdOffsets - 1) / kAdOffsets;
+    // item sub * N + i of nsub * N, which may not fit 32 bits: both parts advance
+    const uint32_t first = blockIdx.x * 4 + wave, stride = gridDim.x * 4;
+    const int32_t dsub = (int32_t)(stride / N), di = (int32_t)(stride % N);
+    int32_t sub = (int32_t)(first / N), i = (int32_t)(first % N);
+    for (; sub < nsub; sub += dsub + (i + di >= N), i = i + di >= N ? i + di - N : i + di) {
         const int32_t e0 = sub * kAdOffsets, e1 = min(ndist, e0 + kAdOffsets);
         const float4 r = S.sx[(int64_t)i * 64 + lane];
         const int bx = __float_as_int(reinterpret_cast<const float *>(S.cbox + kBox * (int64_t)i)[lane & 7]);
