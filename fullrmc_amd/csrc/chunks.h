@@ -10,8 +10,11 @@ namespace frmc {
 constexpr int kNZ = 128;            // counting-sort bins along a column
 constexpr int kBox = 4;             // float4 per chunk box
 
-// words of the scratch header (zeroed before the sort, then the plan)
-enum { M_AMAX = 0, M_NCHUNK = 1, M_PAIRS = 4, M_LO = 8, M_HI = 11, M_PLAN = 16, M_WORDS = 64 };
+// words of the scratch header (zeroed before the sort, then the plan; then the
+// evaluated pairs while they are counted, over kPairWords cache lines: the waves'
+// atomics took 60 us at 13,500 atoms on one word, 20 on 32 words of two lines)
+constexpr int kPairWords = 32, kPairStep = 32;
+enum { M_AMAX = 0, M_NCHUNK = 1, M_LO = 8, M_HI = 11, M_PLAN = 16, M_PAIRS = 64, M_WORDS = M_PAIRS + kPairStep * kPairWords };
 
 // Lower bound of a squared distance from fractional differences known up to
 // half-widths: |b B|^2 = |b L|^2 with B B^T = L L^T (L lower triangular).
@@ -29,7 +32,8 @@ struct ChunkPlan {
     int32_t ortho;        // the off-diagonal entries are zero
 };
 constexpr int kPlanWords = sizeof(ChunkPlan) / 4;
-static_assert(sizeof(ChunkPlan) % 4 == 0 && kPlanWords <= 64 && kPlanWords <= M_WORDS - M_PLAN, "plan size");
+static_assert(M_WORDS <= 1024 + M_PAIRS, "the small sort clears the pair words with 1,024 threads");
+static_assert(sizeof(ChunkPlan) % 4 == 0 && kPlanWords <= 64 && kPlanWords <= M_PAIRS - M_PLAN, "plan size");
 
 // Columns across the first two axes, for n atoms: cross-sections of about the
 // side of a cube of 64 atoms, so that 64 consecutive atoms of a column fill

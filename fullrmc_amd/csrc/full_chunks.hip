@@ -110,7 +110,8 @@ __global__ void __launch_bounds__(256) k_chunk_setup(const float *__restrict__ d
                                                      uint32_t *__restrict__ meta, int32_t *__restrict__ cellcnt,
                                                      int64_t cells, int32_t *__restrict__ counts, int64_t ncounts) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
-    if (t < M_PLAN) meta[t] = 0;
+    for (int64_t i = t; i < M_WORDS; i += stride)
+        if (i < M_PLAN || i >= M_PAIRS) meta[i] = 0;
     for (int64_t i = t; i < cells; i += stride) cellcnt[i] = 0;
     for (int64_t i = t; i < ncounts; i += stride) counts[i] = 0;
     if (t == 0) {
@@ -328,6 +329,7 @@ __global__ void __launch_bounds__(1024) k_chunk_sort_small(const float *__restri
         }
     }
     __syncthreads();
+    if (tid < M_WORDS - M_PAIRS) meta[M_PAIRS + tid] = 0;
     if (tid < M_PLAN) {
         uint32_t v = 0;
         if (tid == M_AMAX) v = amax;
@@ -450,7 +452,6 @@ __device__ __forceinline__ void full_chunks(const ChunkArgs &K, const Basis &B, 
     int32_t *__restrict__ counts = K.counts;
     extern __shared__ float4 lds4[];
     __shared__ int32_t next;
-    __shared__ unsigned long long all_evaluated;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwave = blockDim.x >> 6;
     char *mine = reinterpret_cast<char *>(lds4) + wave * kWaveLds;
     float4 *lxyz = reinterpret_cast<float4 *>(mine);
@@ -460,10 +461,7 @@ __device__ __forceinline__ void full_chunks(const ChunkArgs &K, const Basis &B, 
     const int32_t size = (int32_t)A.size, H = A.g.H, nel = A.nel;
     const int32_t nbins = LDS_HIST ? (lds_intra ? 2 * size : size) : 0;  // inter-molecular bins first
     for (int32_t s = tid; s < nbins; s += blockDim.x) hist[s] = 0;
-    if (tid == 0) {
-        next = 0;
-        all_evaluated = 0;
-    }
+    if (tid == 0) next = 0;
     __syncthreads();
 
     const int32_t N = (int32_t)load_dev(meta + M_NCHUNK);
@@ -693,11 +691,9 @@ __device__ __forceinline__ void full_chunks(const ChunkArgs &K, const Basis &B, 
     if (lost) atomicAdd(&counts[2 * A.size], lost);
     if (EDGE && nre)
         atomicAdd(reinterpret_cast<unsigned long long *>(&counts[2 * A.size + 2]), (unsigned long long)nre);
-    if (K.count_pairs) {  // one atomic per workgroup (one per wave: about 60 us more at 13,500 atoms)
-        if (lane == 0) atomicAdd(&all_evaluated, evaluated * 64ull);
-        __syncthreads();
-        if (tid == 0) atomicAdd(reinterpret_cast<unsigned long long *>(&meta[M_PAIRS]), all_evaluated);
-    }
+    if (K.count_pairs && lane == 0)
+        atomicAdd(reinterpret_cast<unsigned long long *>(&meta[M_PAIRS + kPairStep * (blockIdx.x % kPairWords)]),
+                  evaluated * 64ull);
     if (LDS_HIST) {
         __syncthreads();
         int32_t *dst = K.partial + (int64_t)blockIdx.x * nbins;
@@ -771,7 +767,10 @@ __global__ void __launch_bounds__(256) k_chunk_convert(const int32_t *__restrict
 
 // the number of evaluated pairs to a host word
 __global__ void k_chunk_pairs(const uint32_t *__restrict__ meta, int64_t *pairs) {
-    if (threadIdx.x == 0) *pairs = load_dev(reinterpret_cast<const int64_t *>(meta + M_PAIRS));
+    int64_t sum = 0;
+    for (int w = 0; w < kPairWords; w++)
+        sum += load_dev(reinterpret_cast<const int64_t *>(meta + M_PAIRS + kPairStep * w));
+    if (threadIdx.x == 0) *pairs = sum;
 }
 
 // Bounds of the approximate bin t = (v_sqrt(s) - min) * (1/bin) against the
