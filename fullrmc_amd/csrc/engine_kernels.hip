@@ -1722,6 +1722,17 @@ static bool group_bins_fit(const View &V, int64_t ints) {
     return V.gmaxw > 1 && ints <= 4096ll * V.gmaxw && fixed + 4 * ints <= kGroupLds;
 }
 
+// A commit on a group has one proposal's pairs for all of its blocks' bins, so its
+// line is lower and falls with the atoms, whose tiles are the blocks.  Per commit,
+// in LDS against one atomic per pair (us; 12 A, 0.07 atoms/A^3): 13 atoms, 2,400
+// slots, 3,900 atoms -7.0, 39,000 -3.9, 195,000 -1.9; 4 atoms, 2,400 slots -0.7, -0.7,
+// +1.3; 8 atoms, 8,000 slots -2.3, +0.8, +3.2; 2 atoms, 8,000 slots +2.3, +1.9, +4.5;
+// 26 atoms, 8,000 slots -16, -11, -4.0.
+static bool group_commit_pays(const View &V) {
+    const int64_t ints = slot_ints(V);
+    return group_bins_fit(V, ints) && ints * (V.n + 40000ll) <= 73000000ll * V.gmaxw;
+}
+
 // blocks per proposal of k proposals
 static unsigned group_blocks(const View &V, int32_t k) {
     const unsigned tiles = blocks_for(V.n, kGroupThreads / group_parts(V.gmaxw));
@@ -1892,7 +1903,7 @@ static void launch_k_commit_cell(const View &V, const Inline &I, const CommitCtl
 }
 
 int launch_commit(const View &V, const Inline &I, const CommitCtl &C, hipStream_t st) {
-    if (I.k == 0 && group_bins_fit(V, slot_ints(V))) launch_k_commit_cell<true>(V, I, C, st);
+    if (I.k == 0 && group_commit_pays(V)) launch_k_commit_cell<true>(V, I, C, st);
     else launch_k_commit_cell<false>(V, I, C, st);
     FRMC_CHECK_LAUNCH();
     return FRMC_OK;

@@ -922,3 +922,42 @@ def test_batched_replicas_at_the_edges_of_chunks(k):
         assert (E.accepted, E.tolerated) == (S.accepted, S.tolerated)
         assert E.constraints[0].data["intra"].tobytes() == S.constraints[0].data["intra"].tobytes()
         assert E.constraints[0].data["inter"].tobytes() == S.constraints[0].data["inter"].tobytes()
+
+
+@pytest.mark.parametrize("nbins", [390, 393])  # 3,520 slots of two constraints: counted in LDS; 3,544: directly
+def test_group_commits_on_both_sides_of_their_line(nbins):
+    """Deltas of two-atom groups counted in LDS, accepted moves committed in LDS or by
+    one atomic per pair: the state equals the oracle's."""
+    test_group_windows_match_oracle_at_the_edges_of_blocks(1290, (2,), 7, nbins, "cubic")
+
+
+def test_commits_of_small_groups_in_a_large_box_cost_what_their_pairs_cost():
+    """195,000 atoms in pairs: the commit of a move among bins that fit LDS
+    (14.3 us a launch when it was counted there) takes no longer than among twice
+    the bins, which do not and are counted directly (9.6 us)."""
+    import ctypes
+
+    from fullrmc_amd import _lib
+    n, L = 195000, _lib.lib()
+    rng = np.random.default_rng(5)
+    basis = systems.cubic_basis((n / 0.07) ** (1 / 3))
+    s = dict(real=(rng.random((n, 3)) @ basis.astype(np.float64)).astype(F32),
+             elements=[("O", "Si")[i] for i in rng.integers(0, 2, n)], molecules=(np.arange(n) // 2).astype(np.int32),
+             basis=basis, recip=systems.reciprocal(basis))
+    us = {}
+    for nbins in (1000, 2000):
+        x = ((0.5 + np.arange(nbins)) * (12.0 / nbins)).astype(F32)
+        E = device_engine(s, [PairDistributionConstraint(np.stack([x, 1.0 + 0.1 * np.sin(x)], 1).astype(F32))],
+                          groups=[[i, i + 1] for i in range(0, n, 2)], gen=TranslationGenerator(0.1))
+        E.set_tolerance(20.0)
+        random.seed(1)
+        np.random.seed(1)
+        E.run_device(100, k=16)
+        _lib.check(L.frmc_engine_profile(E._device_engine(16), 1))
+        E.run_device(300, k=16, pull=False)
+        ms, launches = (ctypes.c_double * 4)(), (ctypes.c_int64 * 4)()
+        _lib.check(L.frmc_engine_kernel_times(E._device_engine(16), ms, launches))
+        q = _lib.KERNEL_NAMES.index("k_commit")
+        assert launches[q] > 20
+        us[nbins] = 1e3 * ms[q] / launches[q]
+    assert us[1000] < 1.2 * us[2000], us
