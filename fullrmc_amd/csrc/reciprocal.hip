@@ -8,10 +8,11 @@
 //                order of NumPy's axis-0 sum, so bit-identical to the
 //                constraint's S(Q).  One lane per (p, q); some waves of a
 //                workgroup stage M and G in LDS, the others sum.
-//   k_sq_mfma    the same contraction for k curves at once on the matrix
-//                cores (v_mfma_f32_16x16x4_f32, float32 inputs, float32
+//   k_sq_mfma, k_sq_tiles  the same contraction for k curves at once on the
+//                matrix cores (v_mfma_f32_16x16x4_f32, float32 inputs, float32
 //                accumulation): 32x16 tiles, the r range split over a
-//                workgroup's waves.  Not bit-identical to the sequential sum; its error against a
+//                workgroup's waves, or, for large products, 64x64 tiles with the
+//                range split over blocks.  Not bit-identical to the sequential sum; its error against a
 //                float64 transform is measured.
 //   k_Gr_to_sq / k_gr_to_sq   reciprocal_space.pyx:89-122 / :42-80: one lane
 //                per Q; each term in double (sin of the float32 product q*r,
@@ -21,6 +22,7 @@
 //   k_sq_to_Gr   the transform of reciprocal_space.pyx:131-162 (which
 //                raises for any input there), in double, rounded once.
 #include <algorithm>
+#include <mutex>
 
 #include "frmc_device.h"
 #include "frmc_host.h"
@@ -350,6 +352,114 @@ __global__ void __launch_bounds__(64 * W) k_sq_mfma(const float *__restrict__ G,
     }
 }
 
+// Large products: a 64 x 64 tile of C per block of four waves (each a 32 x 32 quarter
+// as 2 x 2 MFMA tiles), the r range in chunks of kKC staged through LDS, the next
+// chunk's global loads in flight while the current one is multiplied.  The r range
+// is split over gridDim.z blocks (enough blocks to fill the chip at small k);
+// their partial tiles go to a buffer that k_sq_splitsum adds in split order.  Each
+// value loaded is used 64 times, in the 32 x 16 tiles above 16 to 32 times, and
+// a long r range spreads over the chip.
+constexpr int kLP = 64, kLQ = 64, kKC = 64;
+constexpr int kLA = kKC + 2;   // As row stride: fragment reads and row stores hit distinct banks
+constexpr int kLB = kLQ + 16;  // Bs row stride: the two rows a half-wave reads land in disjoint banks
+constexpr int kNA = kLP * kKC / 256, kNB = kKC * kLQ / 256;  // chunk elements per thread
+
+__global__ void __launch_bounds__(256) k_sq_tiles(const float *__restrict__ G, int32_t k, int32_t H,
+                                                 const float *__restrict__ M, int32_t nQ, int32_t kPerSplit,
+                                                 int32_t addOne, float *__restrict__ out, int32_t direct) {
+    __shared__ float As[kLP * kLA];
+    __shared__ float Bs[kKC * kLB];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int wp = w >> 1, wq = w & 1;
+    const int32_t p0 = blockIdx.y * kLP, q0 = blockIdx.x * kLQ;
+    const int32_t kb0 = blockIdx.z * kPerSplit;
+    const int32_t kend = min(H, kb0 + kPerSplit);
+    float ar[kNA], br[kNB];
+    // chunk loads: A 64 rows (p) x kKC r, B kKC r x 64 q; indexes clamped into
+    // the arrays, values past the split's r range (or past k / nQ) unused or zero
+    auto load = [&](int32_t kc0) {
+#pragma unroll
+        for (int i = 0; i < kNA; i++) {
+            const int idx = t + 256 * i;
+            const int32_t ra = kc0 + idx % kKC;
+            const float va = G[(int64_t)min(p0 + idx / kKC, k - 1) * H + min(ra, kend - 1)];
+            ar[i] = ra < kend ? va : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < kNB; i++) {
+            const int idx = t + 256 * i;
+            const int32_t rb = kc0 + idx / kLQ;
+            const float vb = M[(int64_t)min(rb, kend - 1) * nQ + min(q0 + idx % kLQ, nQ - 1)];
+            br[i] = rb < kend ? vb : 0.0f;
+        }
+    };
+    floatx4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (kb0 < kend) load(kb0);
+    for (int32_t kc0 = kb0; kc0 < kend; kc0 += kKC) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kNA; i++) {
+            const int idx = t + 256 * i;
+            As[(idx / kKC) * kLA + idx % kKC] = ar[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kNB; i++) {
+            const int idx = t + 256 * i;
+            Bs[(idx / kLQ) * kLB + idx % kLQ] = br[i];
+        }
+        __syncthreads();
+        if (kc0 + kKC < kend) load(kc0 + kKC);
+#pragma unroll
+        for (int kb = 0; kb < kKC; kb += 4) {
+            float af[2], bf[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) af[i] = As[(wp * 32 + 16 * i + (lane & 15)) * kLA + kb + (lane >> 4)];
+#pragma unroll
+            for (int j = 0; j < 2; j++) bf[j] = Bs[(kb + (lane >> 4)) * kLB + wq * 32 + 16 * j + (lane & 15)];
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    float *dst = direct ? out : out + (int64_t)blockIdx.z * k * nQ;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int32_t q = q0 + wq * 32 + 16 * j + (lane & 15);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int32_t p = p0 + wp * 32 + 16 * i + 4 * (lane >> 4) + v;
+                float x = acc[i][j][v];
+                if (direct && addOne) x = x + 1.0f;
+                if (p < k && q < nQ) dst[(int64_t)p * nQ + q] = x;
+            }
+        }
+}
+
+// S = sum over the splits of the partial products, in split order (+1)
+__global__ void __launch_bounds__(256) k_sq_splitsum(const float *__restrict__ part, int32_t nsplit, int64_t len,
+                                                     int32_t addOne, float *__restrict__ S) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += (int64_t)gridDim.x * blockDim.x) {
+        float x = 0.0f;
+        // eight independent loads in flight, then their adds in order
+        for (int32_t z0 = 0; z0 < nsplit; z0 += 8) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = part[(int64_t)min(z0 + j, nsplit - 1) * len + i];
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (z0 + j < nsplit) x = x + v[j];
+        }
+        S[i] = addOne ? x + 1.0f : x;
+    }
+}
+
 // Curves per wave, by the chains (64 Q of a curve each): one up to two chains per
 // SIMD (128 curves of 1,000 Q: 27.6 us with one, 27.4 with two, and 64 curves
 // 19.3 against 27.3), two up to four (256 curves: 51, 41 and 43 us with one, two
@@ -384,6 +494,46 @@ void launch_sq_mfma(const float *G, int32_t k, int32_t H, const float *M, int32_
         else
             k_sq_mfma<8><<<grid, 512, 0, st>>>(G + p * H, kp, H, M, nQ, addOne, S + p * nQ);
     }
+}
+
+// Which matrix-core kernel takes a shape, and the split of the r range over
+// blocks in the large tiles.  The 32 x 16 tiles, without a second kernel, are better
+// where they nearly fill the chip once and r is neither one chunk nor longer
+// than a workgroup's waves hide (us, 32 x 16 against 64 x 64): 128 curves x 2,000
+// r x 1,000 Q 13.6 and 24, 256 x 2,000 x 1,000 25.0 and 29.6, 16,384 x 2,000 x 16
+// 25.4 and 61.9; and worse elsewhere: 1,000 x 2,000 x 1,000 84 and 69, 512 x 2,000 x
+// 4,000 176 and 126, 4,096 x 200 x 1,000 108 and 35, 2,000 x 8 x 1,000 76 and 10, 64 x
+// 8,000 x 300 43 and 27, 1 x 60,000 x 100 241 and 49.
+struct SqPlan {
+    bool tiles;        // k_sq_tiles
+    int64_t bq, bp;    // its tiles
+    int64_t nsplit;    // parts of the r range, about 1,024 blocks in all
+    int32_t per;       // rows of a part
+};
+
+SqPlan sq_plan(int32_t k, int32_t H, int32_t nQ) {
+    SqPlan P;
+    const int64_t t = (int64_t)((k + kTP - 1) / kTP) * ((nQ + kTQ - 1) / kTQ);
+    P.tiles = H <= 64 || H > 5000 || (nQ > kTQ && (t > 700 || t * H > 1050000));
+    P.bq = (nQ + kLQ - 1) / kLQ;
+    P.bp = (k + kLP - 1) / kLP;
+    const int64_t chunks = (H + kKC - 1) / kKC;
+    P.nsplit = std::max<int64_t>(1, std::min<int64_t>((1024 + P.bq * P.bp - 1) / (P.bq * P.bp), chunks));
+    P.per = (int32_t)(((chunks + P.nsplit - 1) / P.nsplit) * kKC);
+    P.nsplit = (H + P.per - 1) / P.per;
+    return P;
+}
+
+// part: nsplit * k * nQ floats if the r range is split
+void launch_sq_tiles(const SqPlan &P, const float *G, int32_t k, int32_t H, const float *M, int32_t nQ, int32_t addOne,
+                     float *part, float *S, hipStream_t st) {
+    const bool direct = P.nsplit == 1;
+    k_sq_tiles<<<dim3((unsigned)P.bq, (unsigned)P.bp, (unsigned)P.nsplit), 256, 0, st>>>(
+        G, k, H, M, nQ, P.per, addOne, direct ? S : part, direct);
+    const int64_t len = (int64_t)k * nQ;
+    if (!direct)
+        k_sq_splitsum<<<(unsigned)std::min<int64_t>(blocks_for(len, 256), 4096), 256, 0, st>>>(part, (int32_t)P.nsplit,
+                                                                                              len, addOne, S);
 }
 
 // reciprocal_space.pyx:89-122: sq = ones; sq[q] += dr*(sin(q*r)/q)*Gr[r]
@@ -529,21 +679,68 @@ extern "C" int frmc_sq_transform(const float *Gr, int32_t k, int32_t H, const fl
         FRMC_REQUIRE(k <= 65535, "sq_transform: at most 65535 curves per call");
     else
         FRMC_REQUIRE(k <= kMaxCurves, "sq_transform: too many curves per call");
-    FRMC_CHECK_HIP(timer.start(st));
-    if (mode == FRMC_SQ_EXACT) launch_sq_exact(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
-    else launch_sq_mfma(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
-    FRMC_CHECK_LAUNCH();
-    FRMC_CHECK_HIP(timer.stop(st));
+    const SqPlan P = sq_plan(k, H, nQ);
+    float *part = nullptr;
+    if (mode == FRMC_SQ_MFMA && P.tiles && P.nsplit > 1) {
+        const hipError_t e = pool_malloc((void **)&part, sizeof(float) * P.nsplit * k * nQ, st);
+        if (e != hipSuccess) {
+            set_error("hipMallocAsync of the split partials failed: %s", hipGetErrorString(e));
+            return FRMC_ENOMEM;
+        }
+    }
+    hipError_t le = timer.start(st);
+    if (le == hipSuccess) {
+        if (mode == FRMC_SQ_EXACT) launch_sq_exact(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
+        else if (P.tiles) launch_sq_tiles(P, Gr, k, H, sqMatrix, nQ, addOne != 0, part, Sq, st);
+        else launch_sq_mfma(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
+        le = hipGetLastError();
+    }
+    if (le == hipSuccess) le = timer.stop(st);
+    if (part) (void)hipFreeAsync(part, st);
+    if (le != hipSuccess) {
+        set_error("sq_transform failed: %s", hipGetErrorString(le));
+        return FRMC_EHIP;
+    }
     return FRMC_OK;
 }
 
 // ------------------------------------------------- no-allocation variant
 //
-// Neither mode of the transform allocates.  The entry keeps the limit on
-// matrix-core shapes that it has had: the curves' and Q points' tiles of 64 x 64,
-// times as many parts of the r range (of 64 rows or more) as make about 1,024 of
-// them, hold at most 2^22 results.
-constexpr int64_t kNoallocResults = (int64_t)1 << 22;
+// The large matrix-core tiles' split partials in a file-scope device array
+// instead of stream-ordered pool memory, for callers that cannot allocate
+// (code under HIP graph capture, allocation-free serving loops).  Each GPU
+// the library runs on holds its own copy (16 MiB) until the process ends.
+// Every call on a GPU shares that GPU's copy, and the next call overwrites
+// it: calls of such shapes that overlap on one GPU (other streams, other threads)
+// race.
+// k_sq_tiles stores every partial element it owns, so nothing needs clearing.
+constexpr int64_t kSqScratchFloats = (int64_t)1 << 22;
+static __device__ __align__(256) float scratch[kSqScratchFloats];
+
+static std::mutex g_sq_scratch_mu;
+static float *g_sq_scratch[64] = {nullptr};  // device address of scratch, per device
+
+// This device's copy of scratch: its address is taken once per device
+// (with that device current), then reused; host code never uses the
+// symbol itself, which is only a host-side stand-in.
+static int sq_scratch_of_current_device(float **out) {
+    int dev = 0;
+    FRMC_CHECK_HIP(hipGetDevice(&dev));
+    FRMC_REQUIRE(dev >= 0 && dev < 64, "sq_transform_noalloc: device %d out of range", dev);
+    std::lock_guard<std::mutex> lock(g_sq_scratch_mu);
+    if (!g_sq_scratch[dev]) {
+        void *p = nullptr;
+        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        if (e != hipSuccess || !p) {
+            set_error("sq_transform_noalloc: hipGetSymbolAddress of the scratch array failed: %s",
+                      hipGetErrorString(e));
+            return FRMC_EHIP;
+        }
+        g_sq_scratch[dev] = (float *)p;
+    }
+    *out = g_sq_scratch[dev];
+    return FRMC_OK;
+}
 
 extern "C" int frmc_sq_transform_noalloc(const float *Gr, int32_t k, int32_t H, const float *sqMatrix, int32_t nQ,
                                          int addOne, int mode, float *Sq, void *stream) {
@@ -559,16 +756,19 @@ extern "C" int frmc_sq_transform_noalloc(const float *Gr, int32_t k, int32_t H, 
         FRMC_CHECK_LAUNCH();
         return FRMC_OK;
     }
-    const int64_t bq = (nQ + 63) / 64, bp = (k + 63) / 64, chunks = (H + 63) / 64;
     FRMC_REQUIRE(k <= kMaxCurves, "sq_transform_noalloc: too many curves per call");
-    int64_t parts = std::max<int64_t>(1, std::min<int64_t>((1024 + bq * bp - 1) / (bq * bp), chunks));
-    const int64_t per = ((chunks + parts - 1) / parts) * 64;
-    parts = (H + per - 1) / per;
-    FRMC_REQUIRE(parts == 1 || parts * k * nQ <= kNoallocResults,
+    const SqPlan P = sq_plan(k, H, nQ);
+    // the limit of the split partials holds for every shape, also those whose tiles need none
+    const int64_t need = P.nsplit * k * nQ;
+    FRMC_REQUIRE(P.nsplit == 1 || need <= kSqScratchFloats,
                  "sq_transform_noalloc: k=%d, H=%d, nQ=%d is past this entry's limit of matrix-core shapes "
                  "(%lld parts of the r range, %lld results in all, at most %lld): use frmc_sq_transform",
-                 k, H, nQ, (long long)parts, (long long)(parts * k * nQ), (long long)kNoallocResults);
-    launch_sq_mfma(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
+                 k, H, nQ, (long long)P.nsplit, (long long)need, (long long)kSqScratchFloats);
+    float *part = nullptr;
+    if (P.tiles && P.nsplit > 1)
+        if (int rc = sq_scratch_of_current_device(&part)) return rc;
+    if (P.tiles) launch_sq_tiles(P, Gr, k, H, sqMatrix, nQ, addOne != 0, part, Sq, st);
+    else launch_sq_mfma(Gr, k, H, sqMatrix, nQ, addOne != 0, Sq, st);
     FRMC_CHECK_LAUNCH();
     return FRMC_OK;
 }

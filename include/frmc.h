@@ -297,7 +297,11 @@ int frmc_sq_transform(const float *Gr, int32_t k, int32_t H, const float *sqMatr
    under HIP graph capture, allocation-free serving loops).  Same arguments
    and results (bit-identical in both modes).  The matrix-core mode returns
    FRMC_EINVAL for shapes whose r range, split over about 1,024 output tiles
-   of 64 x 64, would give more than 2^22 partial floats. */
+   of 64 x 64, would give more than 2^22 partial floats.  Large products (many
+   output tiles, or more than 5,000 r) keep such partials in a library-owned
+   device array of 2^22 floats (16 MiB) per GPU, held until the process ends:
+   calls of those shapes that overlap on one GPU race.  Other shapes and the
+   exact mode use no scratch. */
 int frmc_sq_transform_noalloc(const float *Gr, int32_t k, int32_t H, const float *sqMatrix, int32_t nQ,
                               int addOne, int mode, float *Sq, void *stream);
 

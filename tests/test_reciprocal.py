@@ -202,3 +202,62 @@ def test_mfma_curves_past_the_rows_of_a_grid(k):
         d = D.empty((1,), F32)  # refused before anything is read
         for f in (_lib.lib().frmc_sq_transform, _lib.lib().frmc_sq_transform_noalloc):
             assert f(d.data_ptr(), k + 1, H, d.data_ptr(), nQ, 1, 1, d.data_ptr(), D.stream()) == 1
+
+
+def _best_time(k, H, nQ, mode):
+    import time
+
+    import torch
+
+    from fullrmc_amd import _lib
+    G, M, S = (torch.ones(s, device="cuda") for s in ((k, H), (H, nQ), (k, nQ)))
+    times = []
+    for _ in range(5):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(10):
+            _lib.check(_lib.lib().frmc_sq_transform(G.data_ptr(), k, H, M.data_ptr(), nQ, 1, mode, S.data_ptr(),
+                                                    torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        times.append((time.perf_counter() - t0) / 10)
+    return min(times)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,H,nQ", [(40, 64, 70), (40, 65, 70), (65, 5000, 33), (65, 5001, 33), (700, 130, 500),
+                                    (701, 130, 511), (737, 130, 513), (257, 2500, 700), (70000, 100, 16),
+                                    (70000, 100, 17), (3, 20001, 5), (2000, 8, 1000)])
+def test_mfma_on_both_sides_of_the_tiles_lines(k, H, nQ):
+    """Shapes around the lines between the two matrix-core kernels (one chunk of r,
+    long r, many tiles, few Q): within float32 rounding, and the no-allocation entry
+    gives the same bits where it takes the shape."""
+    import torch
+
+    from fullrmc_amd import _lib
+    rng = np.random.default_rng(k + H + nQ)
+    G = rng.standard_normal((k, H)).astype(F32)
+    M = rng.standard_normal((H, nQ)).astype(F32)
+    S = grs.sq_transform(G, M, addOne=False, mode="mfma")
+    exact, terms = G.astype(np.float64) @ M.astype(np.float64), np.abs(G).astype(np.float64) @ np.abs(M)
+    assert np.all(np.abs(S - exact) <= (H + 1) * 2.0 ** -24 * terms)
+    dG, dM = torch.from_numpy(G).cuda(), torch.from_numpy(M).cuda()
+    dS = torch.zeros((k, nQ), device="cuda")
+    rc = _lib.lib().frmc_sq_transform_noalloc(dG.data_ptr(), k, H, dM.data_ptr(), nQ, 0, 1, dS.data_ptr(),
+                                              torch.cuda.current_stream().cuda_stream)
+    tiles = -(-k // 64) * -(-nQ // 64)
+    parts = min(-(-1024 // tiles), -(-H // 64))
+    per = -(-(-(-H // 64)) // parts) * 64
+    parts = -(-H // per)
+    assert rc == (0 if parts == 1 or parts * k * nQ <= 2 ** 22 else 1)
+    if rc == 0:
+        torch.cuda.synchronize()
+        assert dS.cpu().numpy().tobytes() == S.tobytes()
+
+
+@pytest.mark.gpu
+def test_mfma_of_many_curves_or_long_ranges_uses_the_chip():
+    """Short r ranges of many curves cost their stores (2,000 curves x 8 r x 1,000 Q
+    took 76 us in small tiles, 10 in large ones), and one curve's long range is spread
+    over the chip (60,000 r 241 us in one workgroup per tile, 49 over all)."""
+    assert _best_time(2000, 8, 1000, 1) < 3 * _best_time(2000, 8, 16, 1)
+    assert _best_time(1, 60000, 100, 1) < 5 * _best_time(1, 5000, 100, 1)
