@@ -231,16 +231,25 @@ __global__ void __launch_bounds__(256 + 64 * kSqLoaders) k_sq_exact(const float 
     Rows R[2];
     fetch(R[0], 0, 0);
     int which = 0;
-    for (int32_t c = 0; c < chunks; c++) {
+    for (int32_t c = 0; c + 1 < chunks; c++) {
         const int ahead = which == 2 ? 0 : which + 1;
 #pragma unroll
         for (int i = 0; i < kSqRows / 16; i++) {
             if (i + 1 < kSqRows / 16) fetch(R[(i + 1) & 1], which, 16 * (i + 1));
-            else fetch(R[0], ahead, 0);  // past the last chunk: read, not used
+            else fetch(R[0], ahead, 0);
             add_then_mul(acc, x, R[i & 1].g, R[i & 1].m);
         }
         which = ahead;
         if (c + 2 < chunks) lds_barrier();
+    }
+    // the last chunk: only the sixteens that hold rows (8 rows, 1,000 curves, 4,000 Q:
+    // 30 us with all of them)
+    const int32_t left = H - (chunks - 1) * kSqRows;
+#pragma unroll
+    for (int i = 0; i < kSqRows / 16; i++) {
+        if (16 * i >= left) break;
+        if (i + 1 < kSqRows / 16) fetch(R[(i + 1) & 1], which, 16 * (i + 1));
+        add_then_mul(acc, x, R[i & 1].g, R[i & 1].m);
     }
 #pragma unroll
     for (int j = 0; j < 16; j++)
@@ -252,6 +261,38 @@ __global__ void __launch_bounds__(256 + 64 * kSqLoaders) k_sq_exact(const float 
             const int32_t pp = p0 + wave * P + p;
             if (pp < k) S[(int64_t)pp * nQ + q0 + lane] = addOne ? acc[p] + 1.0f : acc[p];
         }
+}
+
+// A few rows: one lane per (curve, Q), the row loop as it stands.  Bound by the
+// result's stores; the staging above costs more than sixteen rows save (1,000
+// curves x 4,000 Q: 8 rows 15 us against 23, 32 rows 22 against 25, 40 rows 27 against 28).
+constexpr int kSqShort = 32, kSqT = 256;
+
+__global__ void __launch_bounds__(kSqT) k_sq_short(const float *__restrict__ G, int32_t H, const float *__restrict__ M,
+                                                   int32_t nQ, int32_t addOne, float *__restrict__ S) {
+    __shared__ float gs[kSqShort];
+    const int32_t q = blockIdx.x * kSqT + threadIdx.x;
+    if ((int32_t)threadIdx.x < H) gs[threadIdx.x] = G[(int64_t)blockIdx.y * H + threadIdx.x];
+    __syncthreads();
+    if (q >= nQ) return;
+    const float *m = M + q;
+    float acc = 0.0f;  // as in k_sq_exact
+    int32_t i = 0;
+    // batches of 16 rows: the loads issue together, then the dependent adds
+    for (; i + 16 <= H; i += 16) {
+        float mv[16];
+#pragma unroll
+        for (int j = 0; j < 16; j++) mv[j] = m[(int64_t)(i + j) * nQ];
+#pragma unroll
+        for (int j = 0; j < 16; j++) mv[j] = gs[i + j] * mv[j];
+#pragma unroll
+        for (int j = 0; j < 16; j++) acc = acc + mv[j];
+    }
+    for (; i < H; i++) {
+        const float pr = gs[i] * m[(int64_t)i * nQ];
+        acc = acc + pr;
+    }
+    S[(int64_t)blockIdx.y * nQ + q] = addOne ? acc + 1.0f : acc;
 }
 
 // Matrix-core transform: C (k x nQ) = G (k x H) . M (H x nQ).  A workgroup
@@ -469,7 +510,9 @@ void launch_sq_exact(const float *G, int32_t k, int32_t H, const float *M, int32
     const unsigned bq = (unsigned)((nQ + 63) / 64);
     const int64_t chains = (int64_t)bq * k;
     const int threads = 64 * (4 + kSqLoaders);
-    if (chains <= 2048)
+    if (H <= kSqShort && nQ > 128)  // (at 100 Q most lanes of a block would idle: 60,000 curves x 24 rows 68 us against 43)
+        k_sq_short<<<dim3((unsigned)((nQ + kSqT - 1) / kSqT), (unsigned)k), kSqT, 0, st>>>(G, H, M, nQ, addOne, S);
+    else if (chains <= 2048)
         k_sq_exact<1><<<dim3(bq, (unsigned)((k + 3) / 4)), threads, 0, st>>>(G, k, H, M, nQ, addOne, S);
     else if (chains <= 4096)
         k_sq_exact<2><<<dim3(bq, (unsigned)((k + 7) / 8)), threads, 0, st>>>(G, k, H, M, nQ, addOne, S);

@@ -261,3 +261,25 @@ def test_mfma_of_many_curves_or_long_ranges_uses_the_chip():
     over the chip (60,000 r 241 us in one workgroup per tile, 49 over all)."""
     assert _best_time(2000, 8, 1000, 1) < 3 * _best_time(2000, 8, 16, 1)
     assert _best_time(1, 60000, 100, 1) < 5 * _best_time(1, 5000, 100, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 79])
+@pytest.mark.parametrize("k,nQ", [(1, 129), (5, 128), (40, 700), (65535, 130), (3000, 257)])
+def test_exact_sums_of_few_rows(H, k, nQ):
+    """Few rows, on both sides of the line to the staged form and of its sixteens:
+    the sequential sum bit for bit."""
+    rng = np.random.default_rng(H + k + nQ)
+    G = rng.standard_normal((k, H)).astype(F32)
+    M = rng.standard_normal((H, nQ)).astype(F32)
+    ref = np.zeros((k, nQ), F32)
+    for r in range(H):
+        ref += G[:, r:r + 1] * M[r]
+    assert grs.sq_transform(G, M, addOne=False).tobytes() == ref.tobytes()
+
+
+@pytest.mark.gpu
+def test_exact_sums_of_few_rows_cost_their_stores():
+    """1,000 curves x 4,000 Q: 8 rows 15 us and 64 rows 28; both 28 when the staged form
+    added 64 rows for 8."""
+    assert _best_time(1000, 8, 4000, 0) < 0.8 * _best_time(1000, 64, 4000, 0)
