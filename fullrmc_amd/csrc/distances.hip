@@ -82,6 +82,48 @@ __global__ void __launch_bounds__(256) k_vs_all(const float *__restrict__ coords
     }
 }
 
+// One point against all atoms (k = 1): `per` atoms a thread.  Bound by the
+// coordinates' reads and the results' stores; staged as above, 8,000,000 atoms took 47 us
+// against 21.  The point comes through lane-varying loads (see load_dev; uniform
+// coherent loads past the L1 cache: 30 us).
+constexpr int32_t kPointRows = 1 << 20;  // four atoms a thread beyond
+
+template <bool PBC, bool DIFF>
+__global__ void __launch_bounds__(256) k_point_vs_all(const float *__restrict__ coords, int32_t n,
+                                                      const float *__restrict__ basis, int mode,
+                                                      const int32_t *__restrict__ indexes, int32_t atomIndex,
+                                                      const float *__restrict__ points, int32_t k, int allAtoms,
+                                                      int32_t per, float *__restrict__ out) {
+    const int32_t c = min((int32_t)(threadIdx.x & 63), k - 1);  // 0
+    int32_t from = 0;
+    const float *point = points + c;
+    if (mode == PM_INDEX) {
+        const int32_t a = indexes ? indexes[c] : atomIndex + c;
+        if (a < 0 || a >= n) return;  // out-of-range index: nothing written (host shim rejects it)
+        point = coords + 3 * (int64_t)a;
+        from = allAtoms ? 0 : a;  // reference leaves [0,atomIndex) uninitialised
+    }
+    const float px = point[0], py = point[1], pz = point[2];
+    Basis B;
+    if (PBC) load_basis_dev(basis, B);
+    const int64_t i0 = (int64_t)blockIdx.x * 256 * per + threadIdx.x, i1 = min((int64_t)n, i0 + 256 * (int64_t)per);
+#pragma unroll 4
+    for (int64_t i = i0; i < i1; i += 256) {
+        if (i < from) continue;
+        // pairs_distances.pyx:373-375 / 461-463: diff = point - coords[i]
+        const float dx = px - coords[3 * i], dy = py - coords[3 * i + 1], dz = pz - coords[3 * i + 2];
+        float rx = dx, ry = dy, rz = dz;
+        if (PBC) pbc_real(dx, dy, dz, B, rx, ry, rz);
+        if (DIFF) {
+            out[3 * i] = rx;
+            out[3 * i + 1] = ry;
+            out[3 * i + 2] = rz;
+        } else {
+            out[i] = cr_sqrt(norm2(rx, ry, rz));
+        }
+    }
+}
+
 // Row-wise pairs: from_to_points_differences (diff = to[i]-from[i]),
 // pair_difference_to_point (n=1, diff = p2-p1), point_to_point_distance
 // (n=1, diff = p1-p2, distance).
@@ -122,11 +164,29 @@ static int launch_vs_all(bool diff, const float *coords, int32_t n, const float 
     FRMC_REQUIRE(!isPBC || basis != nullptr, "basis is NULL");
     if (n == 0 || k == 0) return FRMC_OK;
     FRMC_REQUIRE(k <= 65535, "too many points (k=%d > 65535)", k);
+    hipStream_t st = as_stream(stream);
+    if (k == 1) {
+        const int32_t per = n > kPointRows ? 4 : 1;
+        const unsigned blocks = blocks_for(n, 256 * per);
+        if (isPBC && diff)
+            k_point_vs_all<true, true><<<blocks, 256, 0, st>>>(coords, n, basis, mode, indexes, atomIndex, points, k,
+                                                               allAtoms, per, out);
+        else if (isPBC)
+            k_point_vs_all<true, false><<<blocks, 256, 0, st>>>(coords, n, basis, mode, indexes, atomIndex, points, k,
+                                                                allAtoms, per, out);
+        else if (diff)
+            k_point_vs_all<false, true><<<blocks, 256, 0, st>>>(coords, n, basis, mode, indexes, atomIndex, points, k,
+                                                                allAtoms, per, out);
+        else
+            k_point_vs_all<false, false><<<blocks, 256, 0, st>>>(coords, n, basis, mode, indexes, atomIndex, points, k,
+                                                                 allAtoms, per, out);
+        FRMC_CHECK_LAUNCH();
+        return FRMC_OK;
+    }
     // about 4,096 elements per workgroup
     const int32_t nc = k < kVsCols ? k : kVsCols;
     const int32_t rows = 4096 / nc < kVsRows ? (4096 / nc < 1 ? 1 : 4096 / nc) : kVsRows;
     dim3 grid(blocks_for(n, rows), (unsigned)((k + kVsCols - 1) / kVsCols));
-    hipStream_t st = as_stream(stream);
     if (isPBC) {
         if (diff)
             k_vs_all<true, true><<<grid, 256, 0, st>>>(coords, n, basis, mode, indexes, atomIndex, points, k,

@@ -278,3 +278,50 @@ def test_tiles_of_points_and_atoms(sysm, isPBC, n, k):
     ref = refcpu.pairs_distances_to_multi_indexcoords(idx, coords, B, isPBC)
     later = np.arange(n)[:, None] >= idx[None, :]
     assert same(got[later], ref[later])
+
+
+@pytest.mark.parametrize("isPBC", [True, False])
+@pytest.mark.parametrize("n", [2, 255, 256, 257])
+def test_one_point_against_all_atoms(sysm, isPBC, n):
+    """The form of one point: distances and differences around its blocks' edges."""
+    test_tiles_of_points_and_atoms(sysm, isPBC, n, 1)
+    coords = np.ascontiguousarray((sysm["box"] if isPBC else sysm["real"])[:n])
+    for a in (0, n - 1):
+        got = gpd.pairs_differences_to_indexcoords(a, coords, sysm["basis"], isPBC, allAtoms=False)
+        ref = refcpu.pairs_differences_to_indexcoords(a, coords, sysm["basis"], isPBC)
+        assert same(got[a:], ref[a:])
+
+
+def test_one_point_against_many_atoms_costs_its_reads_and_stores():
+    """8,000,000 atoms: one point 21 us, 47 in the tiles of many points; four points
+    68."""
+    import time
+
+    import torch
+
+    from fullrmc_amd import _lib
+    n = 8000000
+    coords, basis = torch.rand((n, 3), device="cuda"), 50.0 * torch.eye(3, device="cuda")
+    idx, out = torch.arange(4, dtype=torch.int32, device="cuda"), torch.empty((n, 4), device="cuda")
+    best = {}
+    for k in (1, 4):
+        times = []
+        for _ in range(6):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(10):
+                _lib.check(_lib.lib().frmc_pairs_distances_to_multi_indexcoords(
+                    idx.data_ptr(), k, coords.data_ptr(), n, basis.data_ptr(), 1, 1, out.data_ptr(),
+                    torch.cuda.current_stream().cuda_stream))
+            torch.cuda.synchronize()
+            times.append(time.perf_counter() - t0)
+        best[k] = min(times)
+    assert best[1] < 0.5 * best[4], best
+    # several atoms a thread, from the point's own row on in the other form
+    n = (1 << 20) + 1025
+    c, b = coords[:n].cpu().numpy(), basis.cpu().numpy()
+    for a in (0, 1 << 20, n - 1):
+        for allAtoms in (True, False):
+            got = gpd.pairs_distances_to_indexcoords(a, c, b, True, allAtoms=allAtoms)
+            ref = refcpu.pairs_distances_to_indexcoords(a, c, b, True)
+            assert same(got if allAtoms else got[a:], ref if allAtoms else ref[a:])
