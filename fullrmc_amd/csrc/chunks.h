@@ -10,11 +10,12 @@ namespace frmc {
 constexpr int kNZ = 128;            // counting-sort bins along a column
 constexpr int kBox = 4;             // float4 per chunk box
 
-// words of the scratch header (zeroed before the sort, then the plan; then the
+// words of the scratch header (zeroed before the sort, then the plan; six 64-bit
+// sums of open boundaries; then the
 // evaluated pairs while they are counted, over kPairWords cache lines: the waves'
 // atomics took 60 us at 13,500 atoms on one word, 20 on 32 words of two lines)
 constexpr int kPairWords = 32, kPairStep = 32;
-enum { M_AMAX = 0, M_NCHUNK = 1, M_LO = 8, M_HI = 11, M_PLAN = 16, M_PAIRS = 64, M_WORDS = M_PAIRS + kPairStep * kPairWords };
+enum { M_AMAX = 0, M_NCHUNK = 1, M_LO = 8, M_HI = 11, M_PLAN = 16, M_SUM = 46, M_PAIRS = 64, M_WORDS = M_PAIRS + kPairStep * kPairWords };
 
 // Lower bound of a squared distance from fractional differences known up to
 // half-widths: |b B|^2 = |b L|^2 with B B^T = L L^T (L lower triangular).
@@ -33,7 +34,7 @@ struct ChunkPlan {
 };
 constexpr int kPlanWords = sizeof(ChunkPlan) / 4;
 static_assert(M_WORDS <= 1024 + M_PAIRS, "the small sort clears the pair words with 1,024 threads");
-static_assert(sizeof(ChunkPlan) % 4 == 0 && kPlanWords <= 64 && kPlanWords <= M_PAIRS - M_PLAN, "plan size");
+static_assert(sizeof(ChunkPlan) % 4 == 0 && kPlanWords <= 64 && kPlanWords <= M_SUM - M_PLAN && M_SUM + 12 <= M_PAIRS, "plan size");
 
 // Columns across the first two axes, for n atoms: cross-sections of about the
 // side of a cube of 64 atoms, so that 64 consecutive atoms of a column fill

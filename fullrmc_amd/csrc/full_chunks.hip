@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(256) k_chunk_setup(const float *__restrict__ d
                                                      int64_t cells, int32_t *__restrict__ counts, int64_t ncounts) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
     for (int64_t i = t; i < M_WORDS; i += stride)
-        if (i < M_PLAN || i >= M_PAIRS) meta[i] = 0;
+        if (i < M_PLAN || i >= M_SUM) meta[i] = 0;
     for (int64_t i = t; i < cells; i += stride) cellcnt[i] = 0;
     for (int64_t i = t; i < ncounts; i += stride) counts[i] = 0;
     if (t == 0) {
@@ -124,37 +124,75 @@ __global__ void __launch_bounds__(256) k_chunk_setup(const float *__restrict__ d
     }
 }
 
-// open boundaries: the coordinates' extent (maxima of the ordered bits and of their complements)
+// Open boundaries: the sort's cells cover mean +- 1.8 standard deviations along
+// each axis, within the extent (a uniform box entirely, at 1.74); atoms past
+// them fall into the cells at the ends.  Over the extent alone one atom far away puts
+// all others into one cell: 50,000 atoms and one at a thousand times their extent
+// 1,312 us a call against 436 (874 for all pairs).
+struct Window {
+    float from, wide;
+};
+__device__ Window sort_window(float lo, float hi, double sum, double squares, int32_t n) {
+    const double mean = sum / n, d = 1.8 * sqrt(fmax(squares / n - mean * mean, 0.0));
+    const float a = fmaxf(lo, (float)(mean - d)), b = fminf(hi, (float)(mean + d));
+    return b > a ? Window{a, b - a} : Window{lo, hi - lo};
+}
+
+__device__ __forceinline__ void add_finite(float x, double &sum, double &squares) {
+    const double v = fabsf(x) < 1e30f ? x : 0.0;
+    sum += v;
+    squares += v * v;
+}
+
+// open boundaries: the coordinates' extent (maxima of the ordered bits and of their
+// complements), and the sums of the sort's window
 __global__ void __launch_bounds__(256) k_chunk_extent(const float *__restrict__ coords, int32_t n,
                                                       uint32_t *__restrict__ meta) {
+    __shared__ uint32_t ext[6];
+    __shared__ double sums[6];
+    if (threadIdx.x < 6) {
+        ext[threadIdx.x] = 0;
+        sums[threadIdx.x] = 0.0;
+    }
+    __syncthreads();
     uint32_t hi[3] = {0, 0, 0}, lo[3] = {0, 0, 0};
+    double sum[3] = {0.0, 0.0, 0.0}, squares[3] = {0.0, 0.0, 0.0};
     for (int32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            const uint32_t u = ordered_bits(coords[3 * (int64_t)i + k]);
+            const float x = coords[3 * (int64_t)i + k];
+            const uint32_t u = ordered_bits(x);
             hi[k] = max(hi[k], u);
             lo[k] = max(lo[k], ~u);
+            add_finite(x, sum[k], squares[k]);
         }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         for (int o = 32; o > 0; o >>= 1) {
             hi[k] = max(hi[k], (uint32_t)__shfl_xor((int)hi[k], o));
             lo[k] = max(lo[k], (uint32_t)__shfl_xor((int)lo[k], o));
+            sum[k] += __shfl_xor(sum[k], o);
+            squares[k] += __shfl_xor(squares[k], o);
         }
         if ((threadIdx.x & 63) == 0) {
-            atomicMax(&meta[M_HI + k], hi[k]);
-            atomicMax(&meta[M_LO + k], lo[k]);
+            atomicMax(&ext[k], lo[k]);
+            atomicMax(&ext[3 + k], hi[k]);
+            atomicAdd(&sums[k], sum[k]);
+            atomicAdd(&sums[3 + k], squares[k]);
         }
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        atomicMax(&meta[M_LO + threadIdx.x], ext[threadIdx.x]);
+        atomicAdd(reinterpret_cast<double *>(meta + M_SUM) + threadIdx.x, sums[threadIdx.x]);
     }
 }
 
-// fraction of coordinate x along axis k in [0, 1]
+// fraction of coordinate x along an axis, in [0, 1] where a window covers it
 template <bool PBC>
-__device__ __forceinline__ float sort_fraction(float x, const uint32_t *__restrict__ meta, int k) {
+__device__ __forceinline__ float sort_fraction(float x, const Window &W) {
     if (PBC) return x - floorf(x);
-    const float lo = from_ordered(~load_dev(meta + M_LO + k)), hi = from_ordered(load_dev(meta + M_HI + k));
-    const float w = hi - lo;
-    return w > 0.0f ? (x - lo) / w : 0.0f;
+    return W.wide > 0.0f ? (x - W.from) / W.wide : 0.0f;
 }
 
 // counting-sort cell of a position's fractions: its column, then its bin along the column
@@ -171,12 +209,21 @@ __global__ void __launch_bounds__(256) k_chunk_count(const float *__restrict__ c
     const int32_t i = blockIdx.x * 256 + threadIdx.x;
     const int32_t m0 = (int32_t)load_dev(meta + M_PLAN + offsetof(ChunkPlan, m0) / 4),
                   m1 = (int32_t)load_dev(meta + M_PLAN + offsetof(ChunkPlan, m1) / 4);
+    __shared__ Window W[3];
+    if (!PBC) {
+        const int k = threadIdx.x;
+        const double *sums = reinterpret_cast<const double *>(meta + M_SUM);
+        if (k < 3)
+            W[k] = sort_window(from_ordered(~load_dev(meta + M_LO + k)), from_ordered(load_dev(meta + M_HI + k)),
+                               load_dev(sums + k), load_dev(sums + 3 + k), n);
+        __syncthreads();
+    }
     float a = 0.0f;
     if (i < n) {
         const float x = coords[3 * (int64_t)i], y = coords[3 * (int64_t)i + 1], z = coords[3 * (int64_t)i + 2];
         if (PBC) a = fmaxf(fmaxf(abs_or_inf(x), abs_or_inf(y)), abs_or_inf(z));
-        const int32_t cell = cell_of(sort_fraction<PBC>(x, meta, 0), sort_fraction<PBC>(y, meta, 1),
-                                     sort_fraction<PBC>(z, meta, 2), m0, m1);
+        const int32_t cell = cell_of(sort_fraction<PBC>(x, W[0]), sort_fraction<PBC>(y, W[1]),
+                                     sort_fraction<PBC>(z, W[2]), m0, m1);
         where[i] = make_int2(cell, atomicAdd(&cellcnt[cell], 1));
     }
     if (!PBC) return;  // the extent gives it
@@ -342,17 +389,15 @@ __global__ void __launch_bounds__(1024) k_chunk_sort_small(const float *__restri
         meta[M_PLAN + tid - 64] = w;
     }
     const int32_t m0 = P.m0, m1 = P.m1, ncol = m0 * m1;
-    float from[3] = {0.f, 0.f, 0.f}, wide[3] = {1.f, 1.f, 1.f};
+    // (over the extent: the sums of the large sort's window would cost 5 us more than they save here)
+    Window W[3] = {{0.f, 1.f}, {0.f, 1.f}, {0.f, 1.f}};
     if (!PBC)
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            from[k] = from_ordered(~ext[k]);
-            wide[k] = from_ordered(ext[3 + k]) - from[k];
+            W[k].from = from_ordered(~ext[k]);
+            W[k].wide = from_ordered(ext[3 + k]) - W[k].from;
         }
-    auto frac = [&](float x, int k) {
-        if (PBC) return x - floorf(x);
-        return wide[k] > 0.0f ? (x - from[k]) / wide[k] : 0.0f;
-    };
+    auto frac = [&](float x, int k) { return sort_fraction<PBC>(x, W[k]); };
     for (int32_t i = tid; i < n; i += 1024) {
         const int32_t c = cell_of(frac(coords[3 * i], 0), frac(coords[3 * i + 1], 1), frac(coords[3 * i + 2], 2), m0, m1);
         where[i] = make_int2(c, atomicAdd(&cell[c], 1));

@@ -163,3 +163,64 @@ def test_few_atoms_of_many_elements(n):
             times.append(time.perf_counter() - t0)
         best[nel] = min(times)
     assert best[64] < 5 * best[2], best
+
+
+@pytest.mark.parametrize("n", [4097, 9001])
+@pytest.mark.parametrize("case", ["far", "offset", "line", "point", "not finite", "two clusters"])
+def test_open_boundaries_of_uneven_extent(n, case):
+    """Open boundaries whose extent says little about where the atoms are: the sort's
+    cells cover the bulk of them, the rest fall into the cells at the ends."""
+    rng = np.random.default_rng(n)
+    coords = rng.random((n, 3)) * 40.0
+    if case == "far":
+        coords[5] = 1e7, -3e5, 2e4
+    elif case == "offset":
+        coords += 5000.0
+    elif case == "line":
+        coords[:, 1:] = 3.0
+    elif case == "point":
+        coords[:] = 1.5
+        coords[: n // 2] += 6.0
+    elif case == "not finite":
+        coords[7, 0], coords[80, 1], coords[900, 2] = np.nan, np.inf, 2e38
+    else:
+        coords[n // 3:] += 3e4
+    coords = coords.astype(F32)
+    mol, elem = (np.arange(n) // 3).astype(np.int32), rng.integers(0, 2, n).astype(np.int32)
+    grid = (2, F32(0.0), F32(9.0), F32(0.03), 300)
+    basis = systems.cubic_basis(40.0)
+    got = gph.full_pairs_histograms_coords(coords, basis, False, mol, elem, *grid)
+    keep = np.all(np.isfinite(coords), axis=1)
+    want = refcpu.full_pairs_histograms_coords(coords[keep], basis, False, mol[keep], elem[keep], *grid, ncores=8)
+    assert got[0].sum() + got[1].sum() > 0
+    assert got[0].tobytes() == want[0].tobytes() and got[1].tobytes() == want[1].tobytes()
+
+
+def test_one_atom_far_away_costs_no_more_than_all_pairs():
+    """50,000 atoms in open boundaries and one of them at a thousand times their extent:
+    436 us a call, 1,312 when the extent alone gave the cells, all pairs 874."""
+    import torch
+    rng = np.random.default_rng(3)
+    n, H, side = 50000, 600, 91.0
+    coords = (rng.random((n, 3)) * side).astype(F32)
+    coords[0] = 1000 * side
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in
+           (coords, systems.cubic_basis(side), np.arange(n, dtype=np.int32) // 3, rng.integers(0, 2, n).astype(np.int32),
+            np.zeros((2, 2, 2, H), F32))]
+    c, b, m, e, out = (t.data_ptr() for t in dev)
+    best = {}
+    for on in (True, False):
+        tuning.set_autotune(on)
+        try:
+            times = []
+            for _ in range(6):
+                torch.cuda.synchronize()
+                t0 = time.perf_counter()
+                _lib.check(_lib.lib().frmc_full_pairs_histograms_coords(
+                    c, n, b, 0, m, e, 2, 0.0, 12.0, 0.02, H, out, out + 16 * H, torch.cuda.current_stream().cuda_stream))
+                torch.cuda.synchronize()
+                times.append(time.perf_counter() - t0)
+            best[on] = min(times)
+        finally:
+            tuning.set_autotune(True)
+    assert best[True] < 0.8 * best[False], best
